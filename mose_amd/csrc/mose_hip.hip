@@ -1383,6 +1383,55 @@ static int plan_ghost_fill(mose_ctx* c) {
   return 0;
 }
 
+// Default tiling of a layout: the (shape, k chunk) of least modelled stage time.  A workgroup
+// marches its tile plane by plane, and the planes of a tile are a serial chain (about 6 us each
+// with one workgroup on a CU), so a layout cut into fewer tiles than the device holds workgroups
+// runs at the length of its longest tile: on 33x25x17 cells 32-plane chunks give 8 tiles and a
+// 175 us stage, one-plane chunks 136 tiles and 21 us; on 131x97x75, 12-plane chunks fill the 512
+// resident workgroups exactly once (108 us; 32 planes 193 us, 1 plane 289 us).  A tile of k planes
+// costs k + 2.5 plane times (its prologue loads four planes and forms the face below the first
+// one: 256^3 in one-plane chunks takes 3.1 times the 16-plane stage), and the stage takes as many
+// rounds as the tiles need on the resident workgroups.  Plane time of a shape with the CU full, by
+// the columns a CU then holds (32x16: 1092 us against 1116 us for 32x8 on 256^3, 86 against 101 us
+// on 128x96x80, 42 against 54 us on the 512x256 channel); a 256-thread workgroup alone on its CU
+// takes 0.62 of it (5.8 us against 9.5 us).  FP32-flux and MUSCL-SD layouts keep shape 0, viscous
+// FP64 layouts take the 128-thread patch (three on a CU: 636 against 712 us on 2x128^3).  Viscous
+// FP32-flux layouts keep the 32-plane chunks too: the face below a chunk's first plane is formed
+// by a copy of the face code that rounds differently in FP32, so the chunk would change their
+// results by 8e-8.
+static void pick_tiling(mose_ctx* c, int* shape, int* kchunk) {
+  const int prec = c->cfg.precision == MOSE_PREC_FP32_FLUX ? 1 : 0;
+  const int kcs[] = {1, 2, 3, 4, 6, 8, 10, 12, 16, 20, 24, 32, 48, 64};
+  const bool visc = geo_kind(c) == 2;
+  if (visc && prec == 1) return;
+  double best = 1e300;
+  for (int s = 0; s < NSHAPE; ++s) {
+    if (!shape_compiled(c, s)) continue;
+    if (prec == 1 && s != 0) continue;
+    if (visc && prec == 0 && s != 2 && shape_compiled(c, 2)) continue;
+    c->shape = s;
+    c->tx = kShape[prec][s][0];
+    c->ty = kShape[prec][s][1];
+    const int nt = c->tx * c->ty, per_cu = std::max(resident_per_cu(c, stage_fn(c, 0)), 1);
+    const double full = nt >= 512 ? 0.92 : 1.0, alone = per_cu > 1 ? 0.62 : full;
+    for (int kc : kcs) {
+      int64_t n = 0;
+      int longest = 1;
+      for (const BlockDev& B : c->lay.blocks) {
+        n += (int64_t)((B.ni + c->tx - 1) / c->tx) * ((B.nj + c->ty - 1) / c->ty) * ((B.nk + kc - 1) / kc);
+        longest = std::max(longest, std::min(kc, B.nk));
+      }
+      const int64_t ncu = std::max(c->ncu, 1), slots = ncu * per_cu;
+      const double t = (longest + 2.5) * (n <= ncu ? alone : full * (double)((n + slots - 1) / slots));
+      if (t < best * 0.999) {
+        best = t;
+        *shape = s;
+        *kchunk = kc;
+      }
+    }
+  }
+}
+
 // ============================================================================= C ABI
 extern "C" {
 
@@ -1518,10 +1567,11 @@ int mose_finalize(mose_ctx* c) {
     hipLaunchKernelGGL(k_fill, dim3(launch_blocks(c->npool)), dim3(256), 0, c->stream, c->d_beta, c->npool, 1.0);
     HIPCHK(c, hipStreamSynchronize(c->stream));
   }
-  // tiling: default shape 0, 32-plane chunks, XCD-aware order, persistent launch;
+  // tiling: shape and chunk by the cost rule (pick_tiling), XCD-aware order, persistent launch;
   // MOSE_TILE_SHAPE, MOSE_KCHUNK and MOSE_TILE_XCD (bit 0 order, bit 1 one workgroup per
   // tile) override (mose_autotune picks by measurement)
   int shape = 0, kc = 32, xcd = 1;
+  pick_tiling(c, &shape, &kc);
   if (const char* e = getenv("MOSE_TILE_SHAPE")) shape = shape_compiled(c, atoi(e)) ? atoi(e) : 0;
   if (const char* e = getenv("MOSE_KCHUNK")) kc = std::max(1, atoi(e));
   if (const char* e = getenv("MOSE_TILE_XCD")) xcd = atoi(e) & 3;
