@@ -2,15 +2,18 @@
 //
 // One explicit step (Explicit_Step, src/lib/numerics/time/explicit/Mod_Explicit.f90:10-146)
 // is this launch sequence on one HIP stream, captured once into a hipGraph:
-//   k_begin    iter += 1; dt = CFL time step of the current state; time += dt when
-//              time-accurate; reset the dt accumulator to 1e5     (Mod_Explicit.f90:36-49)
-//   n_rk x { k_ghost   ghost layers of every block face            (Lib_Ghost.f90:11-137)
-//            k_bcface  fluxes of the non-connection boundary faces (Mod_BC_Fluxes.f90:10-218)
+//   n_rk x { k_ghost   ghost layers of every block face            (Lib_Ghost.f90:11-137); the
+//                      first one also starts the step (begin_step): iter += 1; dt = CFL time
+//                      step of the current state; time += dt when time-accurate; reset the dt
+//                      accumulator to 1e5                          (Mod_Explicit.f90:36-49)
+//            k_bcface  fluxes of the non-connection boundary faces (Mod_BC_Fluxes.f90:10-218),
+//                      in the ghost fill's launch where the two are independent
 //            k_stage   all other face fluxes (Mod_Fluxes.f90:46-209) and the SSP-RK stage
 //                      update (Lib_Newstate.f90:134-160) fused; the last stage also
 //                      produces the residual-norm partial sums (Mod_Diagnostic.f90:13-50)
 //                      and, from the state it writes, the CFL time step of the next step
 //                      (Compute_dt, Mod_dt.f90:10-107: wave-shuffle min, one atomic per wave) }
+// and once per call, for its last step:
 //   k_normfin  fixed-order sum of the partials, sqrt                (Mod_Explicit.f90:111-112)
 // k_dt computes the CFL time step directly when the state did not come from a step.
 // Copy_State (PO = P) needs no pass: U^n stays in its own buffer while the stages run.
@@ -105,17 +108,6 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_dt(DtArgs a) {
   for (int o = 32; o > 0; o >>= 1) mymin = fmin(mymin, __shfl_xor(mymin, o, 64));
   if ((tid & 63) == 0 && mymin < 1e300)
     atomicMin(a.dtmin, (unsigned long long)__double_as_longlong(mymin));
-}
-
-// Start of a step: iter += 1, take the CFL time step computed from the current state (by
-// the previous step's last stage or by k_dt), time += dt when time-accurate, and reset the
-// accumulator (dtglobal = 1e5, Mod_Explicit.f90:36-49) for this step's last stage.
-__global__ void k_begin(unsigned long long* dtmin, int* iter, double* scal, int time_accurate) {
-  *iter += 1;
-  const double dt = __longlong_as_double((long long)*dtmin);
-  scal[S_DT] = dt;
-  if (time_accurate) scal[S_TIME] += dt;
-  *dtmin = (unsigned long long)__double_as_longlong(1e5);
 }
 
 __global__ void k_dtreset(unsigned long long* dtmin) {
@@ -348,7 +340,7 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_irs_update(StageArgs a, int
       }
     }
     if constexpr (LAST) {   // fixed-order reduction over the workgroup
-      __shared__ double sW[kMaxTileThreads / 64][5];
+      __shared__ double sW[kMaxTileThreads / 64][5], sDt[kMaxTileThreads / 64];
       const int lane = tid & 63, wave = tid >> 6, nw = (int)(blockDim.x / 64);
 #pragma unroll
       for (int v = 0; v < 5; ++v) {
@@ -363,7 +355,12 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_irs_update(StageArgs a, int
         a.partials[5 * (int64_t)t + tid] = tot;
       }
       for (int o = 32; o > 0; o >>= 1) dtmin_t = fmin(dtmin_t, __shfl_xor(dtmin_t, o, 64));
-      if (lane == 0 && dtmin_t < 1e300) atomicMin(a.dtmin, (unsigned long long)__double_as_longlong(dtmin_t));
+      if (lane == 0) sDt[wave] = dtmin_t;
+      __syncthreads();
+      if (tid == 0) {      // one atomic a tile (all go to one address)
+        for (int w = 1; w < nw; ++w) dtmin_t = fmin(dtmin_t, sDt[w]);
+        if (dtmin_t < 1e300) atomicMin(a.dtmin, (unsigned long long)__double_as_longlong(dtmin_t));
+      }
       __syncthreads();
     }
   }
@@ -432,71 +429,8 @@ __global__ void __launch_bounds__(256) k_normfin(const double* partials, int nti
   if (tid < 5) scal[S_NORM + tid] = sqrt(red[0][tid]);
 }
 
-// Ghost layers (Fill_Ghost_Cell, Lib_Ghost.f90:11-137) on the conserved SoA state.
-// Copies (101/201 Ghost_Connection, zero-gradient) move conserved values, which equal the
-// primitive copies of the reference exactly; extrapolation (Ghost_Extrapolate) and the
-// symmetry mirror (Ghost_Symmetry) act on primitive variables as in the reference.
-// The records of one launch are independent: a record that reads a ghost cell written by an
-// earlier record runs in a later launch (phase), and one that reads a ghost cell written by a
-// later record reads it from arc, the values at the end of the previous fill (narc cells).
-__global__ void __launch_bounds__(256) k_ghost(const GhostOp* __restrict__ ops, int nops, double* U,
-                                               int64_t N, double gam, const double* __restrict__ arc,
-                                               int64_t narc) {
-  const double gm1 = gam - 1.0, rgm1 = 1.0 / gm1;
-  for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < nops; q += gridDim.x * blockDim.x) {
-    const GhostOp op = ops[q];
-    const int64_t d1 = op.b - op.s, d2 = op.b - 2 * op.s;
-    auto rd = [&](int v, int64_t cell, int slot) { return slot >= 0 ? arc[v * narc + slot] : U[v * N + cell]; };
-    if (op.type == G_COPY) {
-#pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        const double a1 = rd(v, op.src1, op.a1), a2 = rd(v, op.src2, op.a2);
-        U[v * N + d1] = a1;
-        U[v * N + d2] = a2;
-      }
-    } else if (op.type == G_ZG) {
-#pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        const double x = U[v * N + op.b];
-        U[v * N + d1] = x;
-        U[v * N + d2] = x;
-      }
-    } else if (op.type == G_EXTRAP) {
-      double u[5], Pb[5], P1[5], P2[5], G1[5], G2[5];
-#pragma unroll
-      for (int v = 0; v < 5; ++v) u[v] = U[v * N + op.b];
-      cons2prim(u, gm1, Pb);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) u[v] = rd(v, op.b + op.s, op.a1);
-      cons2prim(u, gm1, P1);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) u[v] = rd(v, op.b + 2 * op.s, op.a2);
-      cons2prim(u, gm1, P2);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        G1[v] = 3.0 * Pb[v] - 3.0 * P1[v] + P2[v];
-        G2[v] = 3.0 * G1[v] - 3.0 * Pb[v] + P1[v];
-      }
-      prim2cons(G1, rgm1, u);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) U[v * N + d1] = u[v];
-      prim2cons(G2, rgm1, u);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) U[v * N + d2] = u[v];
-    } else {   // G_SYM: first layer only
-      double u[5], P[5];
-#pragma unroll
-      for (int v = 0; v < 5; ++v) u[v] = U[v * N + op.b];
-      cons2prim(u, gm1, P);
-      const double un = P[1] * op.n[0] + P[2] * op.n[1] + P[3] * op.n[2];
-      P[1] -= 2.0 * un * op.n[0];
-      P[2] -= 2.0 * un * op.n[1];
-      P[3] -= 2.0 * un * op.n[2];
-      prim2cons(P, rgm1, u);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) U[v * N + d1] = u[v];
-    }
-  }
+__global__ void __launch_bounds__(256) k_ghost(GhostArgs g) {
+  ghost_ops(g, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
 }
 
 // blk%P (AoS primitive, padded, Fortran order) <-> conserved SoA pool.
@@ -634,8 +568,10 @@ struct mose_ctx {
   double* d_geo = nullptr;
   Tile* d_tiles = nullptr;
   GhostOp* d_ghost = nullptr;                 // ghost records in bc order (the adjoint's transpose)
-  GhostOp* d_ghostp = nullptr;                // the same grouped by fill phase
+  GhostRec* d_ghostp = nullptr;               // the same grouped by fill phase
+  double* d_gnrm = nullptr;                   // mirror normals of its symmetry records
   std::vector<int> gphase;                    // phase p: records [gphase[p], gphase[p+1]) of d_ghostp
+  bool bc_indep = false;                      // boundary-face fluxes read no ghost cell
   int64_t* d_garc_cell = nullptr;             // archived ghost cells (previous-fill values)
   double* d_garc = nullptr;
   int64_t narc = 0;
@@ -732,11 +668,43 @@ static void enqueue_garc_save(mose_ctx* c, const double* U) {
                        c->narc, c->d_garc);
 }
 
-static int enqueue_ghost(mose_ctx* c, double* U) {
-  for (size_t p = 0; p + 1 < c->gphase.size(); ++p) {
+static GhostArgs ghost_args(mose_ctx* c, double* U, int first, int n, bool begin) {
+  GhostArgs g{};
+  g.ops = c->d_ghostp + first; g.nrm = c->d_gnrm; g.nops = n; g.U = U; g.N = c->npool; g.gam = c->cfg.gamma;
+  g.arc = c->d_garc; g.narc = c->narc;
+  if (begin) {
+    g.dtmin = c->d_dtmin; g.iter = c->d_iter; g.scal = c->d_scal; g.time_accurate = c->cfg.time_accurate;
+  }
+  return g;
+}
+
+// Boundary-face fluxes of the stage input a; gh.nblk workgroups of the launch fill ghosts.
+static void launch_bcface(mose_ctx* c, const StageArgs& a, GhostArgs gh) {
+  const int p = c->cfg.precision == MOSE_PREC_FP32_FLUX ? 1 : 0;
+  const int n = (int)c->lay.bcfaces.size();
+  BcFn fn = ktable().bc[p][c->cfg.limiter][c->cfg.riemann];
+  StageArgs aa = a;
+  const BcFace* faces = c->d_bcfaces;
+  void* args[] = {&aa, &faces, (void*)&n, &gh};
+  (void)hipLaunchKernel((const void*)fn, dim3(gh.nblk + launch_blocks(n)), dim3(256), args, 0, c->stream);
+}
+
+// Ghost fill of U (begin: also the start of a step).  With bc, the boundary-face fluxes of that
+// stage input are solved in the first launch where they are independent of the fill; returns
+// whether they were.
+static bool enqueue_ghost(mose_ctx* c, double* U, bool begin = false, const StageArgs* bc = nullptr) {
+  bool bc_done = false;
+  const int np = (int)c->gphase.size() - 1;
+  for (int p = 0; p < np; ++p) {
     const int n = c->gphase[p + 1] - c->gphase[p];
-    hipLaunchKernelGGL(k_ghost, dim3(launch_blocks(n)), dim3(256), 0, c->stream, c->d_ghostp + c->gphase[p], n, U,
-                       c->npool, c->cfg.gamma, c->d_garc, c->narc);
+    GhostArgs g = ghost_args(c, U, c->gphase[p], n, begin && p == 0);
+    if (p == 0 && bc && c->bc_indep && !c->lay.bcfaces.empty()) {
+      g.nblk = launch_blocks(n);
+      launch_bcface(c, *bc, g);
+      bc_done = true;
+    } else {
+      hipLaunchKernelGGL(k_ghost, dim3(launch_blocks(n)), dim3(256), 0, c->stream, g);
+    }
   }
   enqueue_garc_save(c, U);
   if (c->d_beta) {
@@ -745,7 +713,7 @@ static int enqueue_ghost(mose_ctx* c, double* U) {
     SdArgs sa{c->d_pres, c->d_beta, c->d_tiles, c->d_blocks, c->npool, (int)c->lay.tiles.size(), c->tx, c->cfg.gamma};
     hipLaunchKernelGGL(k_sd, dim3(sa.ntiles), dim3(c->tx * c->ty), 0, c->stream, sa);
   }
-  return 0;
+  return bc_done;
 }
 
 static StageArgs stage_args(mose_ctx* c, const double* Uin, const double* Un, double* Uout, double rkc) {
@@ -785,8 +753,9 @@ static void launch_stage(mose_ctx* c, StageFn fn, StageArgs a) {
   (void)hipLaunchKernel((const void*)fn, dim3(std::max(grid, 1)), dim3(c->tx * c->ty), args, 0, c->stream);
 }
 
-// Boundary-face fluxes of the stage input (the BC_Fluxes pass), before the stage kernel.
-static void enqueue_bcfaces(mose_ctx* c, const StageArgs& a) {
+// Boundary-face fluxes of the stage input (the BC_Fluxes pass), before the stage kernel; done:
+// the inviscid ones were solved with the ghost fill.
+static void enqueue_bcfaces(mose_ctx* c, const StageArgs& a, bool done) {
   const int nv = (int)c->lay.vfaces.size();
   if (nv > 0) {   // viscous flux of the connection faces
     StageArgs av = a;
@@ -795,14 +764,7 @@ static void enqueue_bcfaces(mose_ctx* c, const StageArgs& a) {
     const void* fn = c->cfg.precision == MOSE_PREC_FP32_FLUX ? (const void*)k_viscbc<float> : (const void*)k_viscbc<double>;
     (void)hipLaunchKernel(fn, dim3(launch_blocks(nv)), dim3(256), vargs, 0, c->stream);
   }
-  const int n = (int)c->lay.bcfaces.size();
-  if (n == 0) return;
-  const int p = c->cfg.precision == MOSE_PREC_FP32_FLUX ? 1 : 0;
-  BcFn fn = ktable().bc[p][c->cfg.limiter][c->cfg.riemann];
-  StageArgs aa = a;
-  const BcFace* faces = c->d_bcfaces;
-  void* args[] = {&aa, &faces, (void*)&n};
-  (void)hipLaunchKernel((const void*)fn, dim3(launch_blocks(n)), dim3(256), args, 0, c->stream);
+  if (!done && !c->lay.bcfaces.empty()) launch_bcface(c, a, GhostArgs{});
 }
 
 // stage-kernel geometry kind: 0 rectilinear, 1 general metrics, 2 rectilinear viscous
@@ -907,16 +869,12 @@ static void enqueue_irs(mose_ctx* c, const StageArgs& a, bool last) {
 // One explicit step enqueued on the context stream (no host synchronisation).  The CFL
 // time step of the next step is produced by the last RK stage from the state it writes.
 static int enqueue_step(mose_ctx* c) {
-  const int nt = (int)c->lay.tiles.size();
-  hipLaunchKernelGGL(k_begin, dim3(1), dim3(1), 0, c->stream, c->d_dtmin, c->d_iter, c->d_scal,
-                     c->cfg.time_accurate);
   const int nrk = c->cfg.n_rk;
   for (int s = 1; s <= nrk; ++s) {
     double* in = (s == 1) ? c->U[0] : c->U[s - 1];
     double* out = (s == nrk) ? (nrk == 1 ? c->U[1] : c->U[0]) : c->U[s];
-    enqueue_ghost(c, in);
     StageArgs a = stage_args(c, in, c->U[0], out, kRK[nrk - 1][s - 1]);
-    enqueue_bcfaces(c, a);
+    enqueue_bcfaces(c, a, enqueue_ghost(c, in, s == 1, &a));
     if (c->cfg.irs_beta > 0.0 || c->cfg.prim_vars) {
       StageArgs r = a;
       r.irs_scale = c->cfg.prim_vars ? 0 : 1;
@@ -930,7 +888,6 @@ static int enqueue_step(mose_ctx* c) {
     const int64_t n = 5 * c->npool;
     hipLaunchKernelGGL(k_copy, dim3(launch_blocks(n)), dim3(256), 0, c->stream, c->U[1], c->U[0], n);
   }
-  hipLaunchKernelGGL(k_normfin, dim3(1), dim3(256), 0, c->stream, c->d_partials, nt, c->d_scal);
   return 0;
 }
 
@@ -1316,9 +1273,8 @@ static void enqueue_vjp(mose_ctx* c, bool geometry = false, double* U = nullptr)
 static void enqueue_residual(mose_ctx* c) {
   const int64_t n5 = 5 * c->npool;
   hipLaunchKernelGGL(k_fill, dim3(launch_blocks(n5)), dim3(256), 0, c->stream, c->Rbuf, n5, 0.0);
-  enqueue_ghost(c, c->U[0]);
   StageArgs a = stage_args(c, c->U[0], c->U[0], c->U[1], 0.0);
-  enqueue_bcfaces(c, a);
+  enqueue_bcfaces(c, a, enqueue_ghost(c, c->U[0], false, &a));
   launch_stage(c, stage_fn(c, 2), a);
 }
 
@@ -1365,15 +1321,33 @@ static int plan_ghost_fill(mose_ctx* c) {
     }
     np = std::max(np, phase[q] + 1);
   }
-  std::vector<GhostOp> sorted;
+  std::vector<GhostRec> sorted;
+  std::vector<double> nrm;
   sorted.reserve(n);
   c->gphase.assign(1, 0);
   for (int p = 0; p < np; ++p) {
-    for (int q = 0; q < n; ++q)
-      if (phase[q] == p) sorted.push_back(ops[q]);
+    for (int q = 0; q < n; ++q) {
+      if (phase[q] != p) continue;
+      const GhostOp& op = ops[q];
+      GhostRec r{(int)op.b, (int)op.s, (int)op.src1, (int)op.src2, op.type, op.a1, op.a2, 0};
+      if (op.type == G_SYM) {
+        r.nrm = (int)(nrm.size() / 3);
+        nrm.insert(nrm.end(), op.n, op.n + 3);
+      }
+      sorted.push_back(r);
+    }
     c->gphase.push_back((int)sorted.size());
   }
-  if (upload(c, &c->d_ghostp, sorted)) return c->err.code;
+  if (upload(c, &c->d_ghostp, sorted) || upload(c, &c->d_gnrm, nrm)) return c->err.code;
+  // the boundary fluxes that read their cell's inner neighbour read a ghost cell (the opposite
+  // face's) in a block one cell thick: they then wait for the fill
+  c->bc_indep = true;
+  for (const BlockDev& B : c->lay.blocks) {
+    const int n3[3] = {B.ni, B.nj, B.nk};
+    for (int f = 0; f < 6; ++f)
+      if (n3[f / 2] < 2 && (B.bct[f] == F_SYM || B.bct[f] == F_INFLOW || B.bct[f] == F_INLET || B.bct[f] == F_OUTFLOW))
+        c->bc_indep = false;
+  }
   c->narc = (int64_t)cells.size();
   if (c->narc > 0) {
     if (upload(c, &c->d_garc_cell, cells)) return c->err.code;
@@ -1649,6 +1623,9 @@ int mose_advance(mose_ctx* c, int32_t nsteps, double* time_out, double* norms) {
   int s = 0;
   for (; s + kStepsPerGraph <= nsteps; s += kStepsPerGraph) HIPCHK(c, hipGraphLaunch(c->gexec_n, c->stream));
   for (; s < nsteps; ++s) HIPCHK(c, hipGraphLaunch(c->gexec, c->stream));
+  // the norms of the last step (those of the steps before it are not observable)
+  if (nsteps > 0)
+    hipLaunchKernelGGL(k_normfin, dim3(1), dim3(256), 0, c->stream, c->d_partials, (int)c->lay.tiles.size(), c->d_scal);
   int rc = sync_and_check(c);
   double sc[S_COUNT];
   HIPCHK(c, hipMemcpy(sc, c->d_scal, sizeof sc, hipMemcpyDeviceToHost));
@@ -1714,7 +1691,7 @@ int mose_time_kernels(mose_ctx* c, int32_t nrep, double ms[4]) {
         else if (which == 1) enqueue_ghost(c, c->U[0]);
         else {
           StageArgs sa = stage_args(c, c->U[0], c->U[0], c->U[1], 0.25);
-          if (which == 2) enqueue_bcfaces(c, sa);
+          if (which == 2) enqueue_bcfaces(c, sa, false);
           launch_stage(c, stage_fn(c, which == 2 ? 0 : 1), sa);
         }
       }
@@ -2118,9 +2095,8 @@ static void enqueue_fixed_step(mose_ctx* c, double* Un, double* Unext, int upto 
   for (int s = 1; s <= last; ++s) {
     double* in = s == 1 ? Un : c->U[s - 1];
     double* out = s == nrk ? Unext : c->U[s];
-    enqueue_ghost(c, in);
     StageArgs a = stage_args(c, in, Un, out, kRK[nrk - 1][s - 1]);
-    enqueue_bcfaces(c, a);
+    enqueue_bcfaces(c, a, enqueue_ghost(c, in, false, &a));
     launch_stage(c, stage_fn(c, 0), a);
   }
 }
@@ -2316,7 +2292,7 @@ void mose_destroy(mose_ctx* c) {
                   c->d_ghost, c->d_bcfaces, c->d_vfaces, c->d_vbuf, c->d_bcbuf, c->d_facebc, c->d_scal, c->d_partials, c->d_dtloc, c->d_dtmin, c->d_err,
                   c->d_iter, c->d_tq, c->d_Rbar, c->d_W, c->d_BB, c->d_Pbar, c->d_Pp, c->d_segs, c->d_grows, c->d_gents,
                   c->d_GF, c->d_GL, c->d_BG, c->d_GE, c->d_IB, c->d_VW, c->d_VB, c->d_beta, c->d_pres, c->d_ghostp,
-                  c->d_garc_cell, c->d_garc, c->d_rs1, c->d_irsg, c->d_gP, c->d_lam0, c->d_lam1, c->d_Dq,
+                  c->d_garc_cell, c->d_garc, c->d_gnrm, c->d_rs1, c->d_irsg, c->d_gP, c->d_lam0, c->d_lam1, c->d_Dq,
                   c->d_apart, c->d_ares, c->d_icell, c->d_VBC, c->d_Tp, c->d_vbt, c->d_vbrow, c->d_vbent, c->d_volq,
                   c->d_upart, c->d_ke, c->d_mu, c->d_icbeg, c->d_vfbeg, c->d_vfi, c->d_vtiles, c->d_vghost, c->d_VPb};
   for (void* p : bufs)

@@ -67,12 +67,19 @@ __device__ __forceinline__ void prim_at(const double* __restrict__ U, unsigned N
 }
 
 // Boundary faces of non-connection type (BC_Fluxes, Mod_BC_Fluxes.f90:10-218): one thread
-// per boundary face cell; the flux per unit area goes to bcbuf.
+// per boundary face cell; the flux per unit area goes to bcbuf.  The first gh.nblk workgroups of
+// the launch fill ghost cells instead (ghost_ops): the boundary fluxes read a boundary cell and
+// its inner neighbour only, so the two are independent where every such neighbour is an
+// interior cell (512x256 channel: fill 13.2 us and fluxes 11.6 us in two launches, 17.5 us in one).
 template <int LIM, int RS, typename FT>
-__global__ void __launch_bounds__(256) k_bcface(StageArgs a, const BcFace* __restrict__ faces, int nfaces) {
+__global__ void __launch_bounds__(256) k_bcface(StageArgs a, const BcFace* __restrict__ faces, int nfaces, GhostArgs gh) {
+  if ((int)blockIdx.x < gh.nblk) {
+    ghost_ops(gh, blockIdx.x * blockDim.x + threadIdx.x, gh.nblk * blockDim.x);
+    return;
+  }
   const double gm1 = a.gam - 1.0;
   const GasT<FT> g{FT(a.gam), FT(gm1), FT(1.0 / gm1), FT(a.R), FT(a.gam * a.R / gm1)};
-  for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < nfaces; q += gridDim.x * blockDim.x) {
+  for (int q = (blockIdx.x - gh.nblk) * blockDim.x + threadIdx.x; q < nfaces; q += (gridDim.x - gh.nblk) * blockDim.x) {
     const BcFace e = faces[q];
     const BlockDev* Bp = a.blocks + e.b;
     const bool hi = e.f & 1;
@@ -81,11 +88,11 @@ __global__ void __launch_bounds__(256) k_bcface(StageArgs a, const BcFace* __res
     if (bct != F_NONE) {
       FT Pb[5], Pi[5];
       prim_at(a.Uin, (unsigned)a.npool, (unsigned)e.cb, gm1, Pb);
-      prim_at(a.Uin, (unsigned)a.npool, (unsigned)e.cn, gm1, Pi);
       const FT nx = FT(e.n[0]), ny = FT(e.n[1]), nz = FT(e.n[2]);
       if (bct == F_EXTRAP) {
         physical_flux(Pb, nx, ny, nz, g, F);
       } else {
+        prim_at(a.Uin, (unsigned)a.npool, (unsigned)e.cn, gm1, Pi);
         bool done = false;
         if (bct == F_INFLOW) {
           done = inflow405_flux<LIM, RS>(Pb, Pi, hi, nx, ny, nz, a.facebc + 8 * Bp->bcd[e.f], g, F);
@@ -325,22 +332,28 @@ __global__ void __launch_bounds__(TXc* TYc)
   constexpr int NE = TXc + TYc;                  // faces on the high edges of the patch
   static_assert(NH <= NTc && NTc % 64 == 0, "one halo / edge cell per thread at most");
   __shared__ FT sP[5][TYc + 4][TXc + 4];
-  __shared__ FT sSx[5][TYc][TXc + 1];    // [y][x]: "+" i-state of cell x-1 (x = 0: the halo cell)
-  __shared__ FT sSy[5][TYc + 1][TXc];    // [y][x]: "+" j-state of cell y-1
+  // [y][x]: "+" i-state of cell x-1 (x = 0: the halo cell), then the flux of the low i face of
+  // cell x; one thread reads an entry's state and writes its flux
+  __shared__ FT sSx[5][TYc][TXc + 1];
+  __shared__ FT sSy[5][TYc + 1][TXc];    // [y][x]: the same along j, "+" j-state of cell y-1
   __shared__ FT sMx[5][TYc];             // "-" i-state of the halo cell x = TX
   __shared__ FT sMy[5][TXc];             // "-" j-state of the halo cell y = TY
-  __shared__ FT sFi[5][TYc][TXc + 1];    // [y][x]: flux of the low i face of cell x
-  __shared__ FT sFj[5][TYc + 1][TXc];    // [y][x]: flux of the low j face of cell y
+  // flux of the low k face of the thread's own cell: in LDS for the FP64 kernels, whose registers
+  // are full (256^3, 32x16, first stage: 1.071 ms in registers, 1.044 ms here; the "+" k-state
+  // moved too, or alone, 1.056 and 1.063 ms)
+  constexpr bool KLDS = sizeof(FT) == 8 && GEO != 2;
+  __shared__ FT sKm[5][KLDS ? NTc : 1];
   constexpr bool VIS = GEO == 2;
   constexpr int VR = VIS ? 3 : 1, VY = VIS ? TYc + 2 : 1, VX = VIS ? TXc + 2 : 1;
   __shared__ FT sV[VR][4][VY][VX];       // viscous variables, ring over planes k-1, k, k+1
   constexpr int NL = (TXc > TYc ? TXc : TYc) + 3;
   __shared__ FT sRL[2][NL], sLP[2][NL];  // per-tile spacing data along x and y (rectilinear)
   __shared__ double sDel[2][NL], sDL[2][NL];   // node spacing delta and cell length dl along x, y
-  // residual-norm sums: LDS for the FP32-flux kernels (register-bound), registers for FP64
-  // (LDS-bound); reduced in a fixed order either way
-  constexpr bool NLDS = MODE == 1 && sizeof(FT) == 4;
-  __shared__ double sN[5][NLDS ? NTc : 1];
+  // last stage: the thread's residual-norm sums and least CFL time step, in LDS (the registers are
+  // full); reduced in a fixed order
+  __shared__ double sN[5][MODE == 1 ? NTc : 1];
+  __shared__ double sDtT[MODE == 1 ? NTc : 1];
+  __shared__ double sDt[MODE == 1 ? NW : 1];
   static_assert(NTc <= kMaxTileThreads, "tile shape above the helper kernels' launch bound");
 
   const int tid = threadIdx.x, tx = tid % TXc, ty = tid / TXc;
@@ -372,11 +385,10 @@ __global__ void __launch_bounds__(TXc* TYc)
   const int yly = yplus ? -1 : TYc, ylx = ytask ? (yplus ? tid - 64 : tid - 64 - TXc) : 0;
 
   __shared__ int sTile;
-  if (tid == 0) sTile = claim_tile(a.tq, a.nq, a.ntiles);
-  lds_barrier();
+  const bool more = a.ntiles > (int)gridDim.x;      // tiles beyond the workgroups' first ones
   // the tile index is the same for every lane: held in a scalar register, so the tile's block
   // fields, line-table entries and plane offsets are scalar loads and scalar arithmetic
-  for (int t = __builtin_amdgcn_readfirstlane(sTile); t >= 0;) {
+  for (int t = (int)blockIdx.x; t >= 0;) {
     const Tile T = a.tiles[t];
     const BlockDev* __restrict__ Bp = a.blocks + T.b;
     const int ni = Bp->ni, nj = Bp->nj, nk = Bp->nk, sy_ = Bp->sy;
@@ -421,12 +433,12 @@ __global__ void __launch_bounds__(TXc* TYc)
 
     // column queue P(k), P(k+1), P(k+2); "+" k-state of cell k; flux of the k face below;
     // prefetched U(k+3) of the column and U of the next plane's halo cell
-    FT Q0[5], Q1[5], Q2[5], Skp[5], Fkm[5];
-    double Un3[5], Uh[5], nsum[5];
-    double dtmin_t = 1e300;     // last stage: min CFL time step of the new state
+    FT Q0[5], Q1[5], Q2[5], Skp[5], Fkm_[5];
+    double Un3[5], Uh[5];
 #pragma unroll
-    for (int v = 0; v < 5; ++v) { Fkm[v] = FT(0); Skp[v] = FT(0); Un3[v] = 0.0; Uh[v] = 0.0; nsum[v] = 0.0; }
-    if constexpr (NLDS) {
+    for (int v = 0; v < 5; ++v) { Fkm_[v] = FT(0); Skp[v] = FT(0); Un3[v] = 0.0; Uh[v] = 0.0; }
+    if constexpr (MODE == 1) {
+      sDtT[tid] = 1e300;
 #pragma unroll
       for (int v = 0; v < 5; ++v) sN[v][tid] = 0.0;
     }
@@ -626,7 +638,7 @@ __global__ void __launch_bounds__(TXc* TYc)
           for (int v = 0; v < 5; ++v) Lq[v] = sSx[v][ty][tx];
           solve(std::integral_constant<int, 0>{}, 0, i, j, Lq, Smx, F);
 #pragma unroll
-          for (int v = 0; v < 5; ++v) sFi[v][ty][tx] = F[v];
+          for (int v = 0; v < 5; ++v) sSx[v][ty][tx] = F[v];
         }
         if (jface) {
           FT Lq[5], F[5];
@@ -634,7 +646,7 @@ __global__ void __launch_bounds__(TXc* TYc)
           for (int v = 0; v < 5; ++v) Lq[v] = sSy[v][ty][tx];
           solve(std::integral_constant<int, 1>{}, 1, i, j, Lq, Smy, F);
 #pragma unroll
-          for (int v = 0; v < 5; ++v) sFj[v][ty][tx] = F[v];
+          for (int v = 0; v < 5; ++v) sSy[v][ty][tx] = F[v];
         }
         const int e = (tid + 64 * (k & (NW - 1))) % NTc;     // rotating patch-edge assignment
         if (e < NE) {
@@ -651,21 +663,21 @@ __global__ void __launch_bounds__(TXc* TYc)
             solve(std::integral_constant<int, -1>{}, d, fi, fj, Lq, Rq, F);
             if (ex) {
 #pragma unroll
-              for (int v = 0; v < 5; ++v) sFi[v][e][TXc] = F[v];
+              for (int v = 0; v < 5; ++v) sSx[v][e][TXc] = F[v];
             } else {
 #pragma unroll
-              for (int v = 0; v < 5; ++v) sFj[v][TYc][e - TYc] = F[v];
+              for (int v = 0; v < 5; ++v) sSy[v][TYc][e - TYc] = F[v];
             }
           }
         }
         lds_barrier();
 
         // operands of the update of plane k, loaded before the k face is solved so that the
-        // solve covers their latency (rectilinear inviscid stages except the last, whose
-        // residual-norm terms leave no registers for them, and the HLLE++ / HLLC+ solvers,
-        // whose registers are taken too: early, the loads would spill)
+        // solve covers their latency (256^3, first stage: 1.137 ms without; last stage: 1.205 ms
+        // without, 1.154 ms) in the rectilinear inviscid stages, except the HLLE++ / HLLC+
+        // solvers, whose registers are taken: early, the loads would spill
         const unsigned c = cbase + sz * (unsigned)(k + 1);
-        constexpr bool EARLY = GEO == 0 && MODE == 0 && !rs_takes_beta(RS);
+        constexpr bool EARLY = GEO == 0 && MODE != 2 && !rs_takes_beta(RS);
         double un[5], ui[5], dt = 0.0;
         if constexpr (EARLY) {
           if (active) {
@@ -708,9 +720,9 @@ __global__ void __launch_bounds__(TXc* TYc)
           double Racc[5];
 #pragma unroll
           for (int v = 0; v < 5; ++v)
-            Racc[v] = Az * ((double)Fk[v] - (double)Fkm[v]) +
-                      Ax * ((double)sFi[v][ty][tx + 1] - (double)sFi[v][ty][tx]) +
-                      Ay * ((double)sFj[v][ty + 1][tx] - (double)sFj[v][ty][tx]);
+            Racc[v] = Az * ((double)Fk[v] - (double)(KLDS ? sKm[v][tid] : Fkm_[v])) +
+                      Ax * ((double)sSx[v][ty][tx + 1] - (double)sSx[v][ty][tx]) +
+                      Ay * ((double)sSy[v][ty + 1][tx] - (double)sSy[v][ty][tx]);
           if constexpr (MODE == 2) {
             if (a.irs_scale) {
               const double dtc = a.local_dt ? a.dtloc[c] : a.scal[S_DT];
@@ -761,21 +773,23 @@ __global__ void __launch_bounds__(TXc* TYc)
               const int itn = *a.iter + 1;
               if (itn < a.rampa) dtc = dtc * itn / a.rampa;
               if (a.local_dt) a.dtnext[c] = dtc;
-              dtmin_t = fmin(dtmin_t, dtc);
+              sDtT[tid] = fmin(sDtT[tid], dtc);
               double pn[5];
               cons2prim(un, gm1, pn);
 #pragma unroll
               for (int v = 0; v < 5; ++v) {
                 const double dd = P[v] - pn[v];
-                if constexpr (NLDS) sN[v][tid] += dd * dd;
-                else nsum[v] += dd * dd;
+                sN[v][tid] += dd * dd;
               }
             }
 #pragma unroll
             for (int v = 0; v < 5; ++v) a.Uout[v * N + c] = unew[v];
           }
 #pragma unroll
-          for (int v = 0; v < 5; ++v) Fkm[v] = Fk[v];
+          for (int v = 0; v < 5; ++v) {
+            if constexpr (KLDS) sKm[v][tid] = Fk[v];
+            else Fkm_[v] = Fk[v];
+          }
         }
       }
       if (!plane) {      // k = k0-1: only the face k0-1/2
@@ -805,7 +819,10 @@ __global__ void __launch_bounds__(TXc* TYc)
         }
         if (active) {
 #pragma unroll
-          for (int v = 0; v < 5; ++v) Fkm[v] = Fk[v];
+          for (int v = 0; v < 5; ++v) {
+            if constexpr (KLDS) sKm[v][tid] = Fk[v];
+            else Fkm_[v] = Fk[v];
+          }
         }
       }
       // advance the column queue
@@ -816,44 +833,47 @@ __global__ void __launch_bounds__(TXc* TYc)
         for (int v = 0; v < 5; ++v) { Q0[v] = Q1[v]; Q1[v] = Q2[v]; Q2[v] = (FT)p[v]; }
       }
     }
+    // the next tile (every thread has read sTile before the barriers of the planes)
+    if (more && tid == 0) sTile = claim_own(a.tq, a.nq, a.ntiles);
     lds_barrier();
 
     if constexpr (MODE == 1) {   // fixed-order reductions over the workgroup: deterministic
       double tot = 0.0;
-      if constexpr (NLDS) {
-        for (int w = NTc / 2; w > 0; w >>= 1) {
-          if (tid < w) {
+      double dtmin_t = sDtT[tid];
+      for (int w = NTc / 2; w > 0; w >>= 1) {
+        if (tid < w) {
 #pragma unroll
-            for (int v = 0; v < 5; ++v) sN[v][tid] += sN[v][tid + w];
-          }
-          lds_barrier();
-        }
-        if (tid < 5) tot = sN[tid][0];
-      } else {
-        const int lane = tid & 63, wave = tid >> 6;
-        double* sW = reinterpret_cast<double*>(&sSx[0][0][0]);     // face states are dead here
-#pragma unroll
-        for (int v = 0; v < 5; ++v) {
-          double x = nsum[v];
-          for (int o = 32; o > 0; o >>= 1) x += __shfl_down(x, o, 64);
-          if (lane == 0) sW[5 * wave + v] = x;
+          for (int v = 0; v < 5; ++v) sN[v][tid] += sN[v][tid + w];
         }
         lds_barrier();
-        if (tid < 5)
-          for (int w = 0; w < NW; ++w) tot += sW[5 * w + tid];
       }
+      if (tid < 5) tot = sN[tid][0];
       if (tid < 5) a.partials[5 * (int64_t)t + tid] = tot;
+      // one atomic a tile: every one goes to the same address, and 2048 of them (one a wave on the
+      // 512x256 channel) made the last stage 46 us, now 26 us, where the others take 21 us
       for (int o = 32; o > 0; o >>= 1) dtmin_t = fmin(dtmin_t, __shfl_xor(dtmin_t, o, 64));
-      if ((tid & 63) == 0 && dtmin_t < 1e300)
-        atomicMin(a.dtmin, (unsigned long long)__double_as_longlong(dtmin_t));
+      if ((tid & 63) == 0) sDt[tid >> 6] = dtmin_t;
+      lds_barrier();
+      if (tid == 0) {
+        for (int w = 1; w < NW; ++w) dtmin_t = fmin(dtmin_t, sDt[w]);
+        if (dtmin_t < 1e300) atomicMin(a.dtmin, (unsigned long long)__double_as_longlong(dtmin_t));
+      }
       lds_barrier();
     }
-    // every thread has read sTile before the barriers above; claim the next tile
-    if (tid == 0) sTile = claim_tile(a.tq, a.nq, a.ntiles);
-    lds_barrier();
+    if (!more) break;
+    // an empty queue: wave 0 looks at the others
     t = __builtin_amdgcn_readfirstlane(sTile);
+    if (t < 0) {
+      lds_barrier();
+      if (tid < 64) {
+        const int o = claim_other(a.tq, a.nq, a.ntiles);
+        if (tid == 0) sTile = o;
+      }
+      lds_barrier();
+      t = __builtin_amdgcn_readfirstlane(sTile);
+    }
   }
-  if (tid == 0) finish_tiles(a.tq);
+  if (more && tid == 0) finish_tiles(a.tq);
 }
 
 }  // namespace mose

@@ -7,7 +7,7 @@
 #pragma once
 
 typedef void (*StageFn)(mose::StageArgs);
-typedef void (*BcFn)(mose::StageArgs, const mose::BcFace*, int);
+typedef void (*BcFn)(mose::StageArgs, const mose::BcFace*, int, mose::GhostArgs);
 typedef void (*AdjFn)(AdjArgs);
 
 constexpr int NLIM = 6;     // minmod, van Leer, van Albada, first order, MC, superbee
