@@ -1461,15 +1461,13 @@ static int plan_ghost_fill(mose_ctx* c) {
 // the columns a CU then holds (32x16: 1092 us against 1116 us for 32x8 on 256^3, 86 against 101 us
 // on 128x96x80, 42 against 54 us on the 512x256 channel); a 256-thread workgroup alone on its CU
 // takes 0.62 of it (5.8 us against 9.5 us).  FP32-flux and MUSCL-SD layouts keep shape 0, viscous
-// FP64 layouts take the 128-thread patch (three on a CU: 636 against 712 us on 2x128^3).  Viscous
-// FP32-flux layouts keep the 32-plane chunks too: the face below a chunk's first plane is formed
-// by a copy of the face code that rounds differently in FP32, so the chunk would change their
-// results by 8e-8.
+// FP64 layouts take the 128-thread patch (three on a CU: 636 against 712 us on 2x128^3).  FP32-flux
+// layouts take a divisor of 32 planes: the stage then gives the bits of 32-plane chunks
+// (plus_state).
 static void pick_tiling(mose_ctx* c, int* shape, int* kchunk) {
   const int prec = c->cfg.precision == MOSE_PREC_FP32_FLUX ? 1 : 0;
   const int kcs[] = {1, 2, 3, 4, 6, 8, 10, 12, 16, 20, 24, 32, 48, 64};
   const bool visc = geo_kind(c) == 2;
-  if (visc && prec == 1) return;
   double best = 1e300;
   for (int s = 0; s < NSHAPE; ++s) {
     if (!shape_compiled(c, s)) continue;
@@ -1481,6 +1479,7 @@ static void pick_tiling(mose_ctx* c, int* shape, int* kchunk) {
     const int nt = c->tx * c->ty, per_cu = std::max(resident_per_cu(c, stage_fn(c, 0)), 1);
     const double full = nt >= 512 ? 0.92 : 1.0, alone = per_cu > 1 ? 0.62 : full;
     for (int kc : kcs) {
+      if (prec == 1 && kFp32Chunk % kc != 0) continue;
       int64_t n = 0;
       int longest = 1;
       for (const BlockDev& B : c->lay.blocks) {

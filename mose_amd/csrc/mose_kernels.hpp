@@ -250,6 +250,14 @@ __device__ __forceinline__ void begin_step(const GhostArgs& g) {
   *g.dtmin = (unsigned long long)__double_as_longlong(1e5);
 }
 
+// prim2cons with the contraction of the energy written out, so that every copy of the fill gives the
+// same bits (FP32-flux layouts turn a ghost cell one FP64 ulp away into another FP32 value now and
+// then, which marches on to 1e-6 of the state).
+__device__ __forceinline__ void ghost_cons(const double* P, double rgm1, double* U) {
+  U[0] = P[0]; U[1] = P[0] * P[1]; U[2] = P[0] * P[2]; U[3] = P[0] * P[3];
+  U[4] = __builtin_fma(rgm1, P[4], 0.5 * P[0] * (P[1] * P[1] + P[2] * P[2] + P[3] * P[3]));
+}
+
 // The ops q0, q0 + step, ... of one phase.
 __device__ __forceinline__ void ghost_ops(const GhostArgs& g, int q0, int step) {
   if (q0 == 0 && g.dtmin) begin_step(g);
@@ -291,10 +299,10 @@ __device__ __forceinline__ void ghost_ops(const GhostArgs& g, int q0, int step) 
         G1[v] = 3.0 * Pb[v] - 3.0 * P1[v] + P2[v];
         G2[v] = 3.0 * G1[v] - 3.0 * Pb[v] + P1[v];
       }
-      prim2cons(G1, rgm1, u);
+      ghost_cons(G1, rgm1, u);
 #pragma unroll
       for (int v = 0; v < 5; ++v) U[v * N + d1] = u[v];
-      prim2cons(G2, rgm1, u);
+      ghost_cons(G2, rgm1, u);
 #pragma unroll
       for (int v = 0; v < 5; ++v) U[v * N + d2] = u[v];
     } else {   // G_SYM: first layer only
@@ -307,7 +315,7 @@ __device__ __forceinline__ void ghost_ops(const GhostArgs& g, int q0, int step) 
       P[1] -= 2.0 * un * n[0];
       P[2] -= 2.0 * un * n[1];
       P[3] -= 2.0 * un * n[2];
-      prim2cons(P, rgm1, u);
+      ghost_cons(P, rgm1, u);
 #pragma unroll
       for (int v = 0; v < 5; ++v) U[v * N + d1] = u[v];
     }

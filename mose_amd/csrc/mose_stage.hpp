@@ -56,6 +56,28 @@ __device__ __forceinline__ void cell_states_b(const FT* Pm, const FT* P0, const 
   }
 }
 
+// "+" k-state of a cell in FP32, formed outside the march.  The march's face code rounds the slope before
+// it is added (it has two uses there); the copies that form the states below a chunk's first plane
+// fuse the two operations.  The results of FP32 layouts are those of kFp32Chunk-plane chunks: a chunk that
+// starts on a multiple of kFp32Chunk planes keeps the fused form, any other takes the form of the
+// march, so a smaller chunk (a divisor) changes no bit.
+constexpr int kFp32Chunk = 32;
+template <int LIM>
+__device__ __forceinline__ void plus_state(const float* Pm, const float* P0, const float* Pp, float rlm, float rlp,
+                                           float hdl, bool fused, float* Sp) {
+#pragma unroll
+  for (int v = 0; v < 5; ++v) {
+    const float l = limiter<LIM>((Pp[v] - P0[v]) * rlp, (P0[v] - Pm[v]) * rlm);
+    float sum;
+    {
+#pragma clang fp contract(off)
+      const float sg = l * hdl;
+      sum = P0[v] + sg;
+    }
+    Sp[v] = fused ? __builtin_fmaf(l, hdl, P0[v]) : sum;
+  }
+}
+
 template <typename FT>
 __device__ __forceinline__ void prim_at(const double* __restrict__ U, unsigned N, unsigned c, double gm1, FT* P) {
   double u[5], p[5];
@@ -404,6 +426,7 @@ __global__ void __launch_bounds__(TXc* TYc)
     const LineEnt* Lz = a.lines + Bp->line[2];
     const cptr<LineEnt> Lzc = (cptr<LineEnt>)Lz;     // Lz[k] is the same for every lane
     const int k0 = T.k0, k1 = T.k1;
+    const bool offgrid = (k0 - 1) % kFp32Chunk != 0;      // FP32: see plus_state
     const int hgi = T.i0 + hx, hgj = T.j0 + hy;
     const bool hval = tid < NH && hgi <= ni + 2 && hgj <= nj + 2;
     const unsigned hbase = off + (unsigned)(hgi + 1) + (unsigned)sy_ * (unsigned)(hgj + 1);
@@ -451,7 +474,16 @@ __global__ void __launch_bounds__(TXc* TYc)
       const unsigned cm = cbase + sz * (unsigned)(k0);            // cell k0-1
       FT bp = FT(1);
       if constexpr (SDR) bp = FT(beta[k0 >= 2 ? cm : cm + sz]);
-      if constexpr (GEO != 1) {
+      if constexpr (sizeof(FT) == 4) {
+        FT rlm, rlp, hdl;
+        if constexpr (GEO != 1) {
+          rlm = FT(Lzc[k0].rl1); rlp = FT(Lzc[k0 + 1].rl1); hdl = FT(Lzc[k0].lp);
+        } else {
+          rlm = FT(GA(GRLO + 2, cm)); rlp = FT(GA(GRLO + 2, cm + sz)); hdl = FT(0.5 * GA(GDL + 2, cm));
+        }
+        // (cell k0 - 1 may be the first cell of a 32-plane chunk, formed fused by that chunk's copy)
+        plus_state<LIM>(Qm, Q0, Q1, rlm, rlp, hdl, !offgrid || (GEO == 0 && (k0 - 2) % kFp32Chunk == 0), Skp);
+      } else if constexpr (GEO != 1) {
         cell_states_b<LIM, SDR>(Qm, Q0, Q1, FT(Lzc[k0].rl1), FT(Lzc[k0 + 1].rl1), FT(Lzc[k0].lp), FT(1), bp, Sm_, Skp);   // P+(k0-1)
       } else {
         cell_states_b<LIM, SDR>(Qm, Q0, Q1, FT(GA(GRLO + 2, cm)), FT(GA(GRLO + 2, cm + sz)), FT(0.5 * GA(GDL + 2, cm)),
@@ -816,6 +848,8 @@ __global__ void __launch_bounds__(TXc* TYc)
           }
 #pragma unroll
           for (int v = 0; v < 5; ++v) Skp[v] = Sp_[v];
+          if constexpr (sizeof(FT) == 4 && GEO == 0)
+            plus_state<LIM>(Q0, Q1, Q2, FT(Lzc[k + 2].rl1), FT(Lzc[k + 3].rl1), FT(Lzc[k + 2].lp), !offgrid, Skp);
         }
         if (active) {
 #pragma unroll
