@@ -906,7 +906,7 @@ __device__ inline double visc_face_flux_adj(int d, const double (*G)[3], const d
   for (int v = 0; v < 4; ++v)
 #pragma unroll
     for (int x = 0; x < 3; ++x) Gp[v][x] = G[v][x] * M[x];
-  const double temp = Pm[4] / (Pm[0] * Rg);
+  const double irR = rcp_(Pm[0] * Rg), temp = Pm[4] * irR;      // as the primal face flux forms them
   const double mu = sutherland(temp, vis[0], vis[1], vis[2]);
   const double kap = mu * vis[3];
   const double lam = -2.0 / 3.0 * mu;
@@ -940,22 +940,22 @@ __device__ inline double visc_face_flux_adj(int d, const double (*G)[3], const d
   for (int x = 0; x < 3; ++x) Gpb[x][x] += lam * ldb;
   mub += -2.0 / 3.0 * lamb;
   // mu = mu_ref (T/T_ref)^1.5 (T_ref + S)/(T + S): d ln mu / dT = 1.5/T - 1/(T + S)
-  const double tempb = mub * mu * (1.5 / temp - 1.0 / (temp + vis[2]));
-  Pmb[4] += tempb / (Pm[0] * Rg);
-  Pmb[0] -= tempb * temp / Pm[0];
+  const double tempb = mub * mu * (1.5 * rcp_(temp) - rcp_(temp + vis[2]));
+  Pmb[4] += tempb * irR;
+  Pmb[0] -= tempb * temp * irR * Rg;
 #pragma unroll
   for (int v = 0; v < 4; ++v)
 #pragma unroll
     for (int x = 0; x < 3; ++x) Gb[v][x] = Gpb[v][x] * M[x];
-  return mub * mu / vis[0];
+  return mub * mu * rcp_(vis[0]);
 }
 
 // Adjoint of the viscous variables V = (u, v, w, T = p / (rho R)) of a cell added to the
 // adjoint of its primitive state P.
 __device__ __forceinline__ void visc_vars_adj(const double* P, double Rg, const double* Vb, double* Pb) {
-  const double iRr = 1.0 / (P[0] * Rg);
+  const double iRr = rcp_(P[0] * Rg);
   const double T = P[4] * iRr;
-  Pb[0] -= Vb[3] * T / P[0];
+  Pb[0] -= Vb[3] * T * iRr * Rg;
   Pb[1] += Vb[0];
   Pb[2] += Vb[1];
   Pb[3] += Vb[2];
@@ -971,7 +971,7 @@ __device__ __forceinline__ void visc_vars_adj(const double* P, double Rg, const 
 //   k_adj_face    one thread per interior or connection face: recompute the two face states
 //                 and the Riemann flux, reverse them, store the adjoints of the face states
 //                 (the "+" state of the left cell, the "-" state of the right cell);
-//   k_adj_bcface  one thread per non-connection boundary face: reverse of the boundary flux
+//   k_adj_bcface  one thread per boundary face with a flux: reverse of that flux
 //                 into adjoints of the boundary cell and its interior neighbour;
 //   k_adj_cell    one thread per cell (ghost layers included): gathers the reverse of the
 //                 limited slopes of itself and its two neighbours along each direction plus
@@ -1075,6 +1075,12 @@ __device__ __forceinline__ void prim_load(const double* __restrict__ Pp, int64_t
 }
 
 
+// A direction of a block one cell thick with no connection face: no face of it is solved (2-D and
+// 1-D layouts), so its face-state adjoints are neither written nor read.
+__device__ __forceinline__ bool adj_dead_dir(const BlockDev& B, int d) {
+  return (d == 0 ? B.ni : (d == 1 ? B.nj : B.nk)) == 1 && B.bct[2 * d] != F_CONN && B.bct[2 * d + 1] != F_CONN;
+}
+
 template <int LIM, int RS, int GEO>
 __global__ void __launch_bounds__(256) k_adj_face(AdjArgs a) {
   const double gm1 = a.gam - 1.0;
@@ -1150,11 +1156,7 @@ __global__ void __launch_bounds__(256) k_adj_face(AdjArgs a) {
       } else {
         riemann_adj<RS>(PL, PR, n[0], n[1], n[2], g, Fb, Lb, Rb);
       }
-    } else if (GEO == 1 && a.GF) {
-      const size_t np = (size_t)N;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) a.GF[(4 * d + q) * np + c] = 0.0;   // a non-connection face: k_adj_bcface
-    }
+    }      // a non-connection face: k_adj_bcface writes its geometry adjoints
     // every "+" / "-" slot that the cell pass reads is written here (zero when no face uses it)
 #pragma unroll
     for (int v = 0; v < 5; ++v) {
@@ -1166,6 +1168,9 @@ __global__ void __launch_bounds__(256) k_adj_face(AdjArgs a) {
   }
 }
 
+// Faces without a flux are not listed: their adjoints are zero, as the buffers of the geometry adjoints
+// are from the start.  (In the face launch, side by side with k_adj_face, this code's registers would
+// leave that one wave a SIMD in place of four.)
 template <int LIM, int RS>
 __global__ void __launch_bounds__(256) k_adj_bcface(AdjArgs a) {
   const double gm1 = a.gam - 1.0;
@@ -1257,49 +1262,112 @@ __global__ void __launch_bounds__(256) k_adj_cell(AdjArgs a) {
     double acc[5] = {0, 0, 0, 0, 0};
     double rlb[3] = {0, 0, 0}, dlb[3] = {0, 0, 0};
     if (outside <= 1) {
+      // Per direction the slopes of the cell and of its two neighbours.  With general metrics every load
+      // of a direction is issued before the first limiter is reversed: one wait in place of six on
+      // the small layouts that run there (384x192 channel, 22.9 us without, 19.8 us).  Rectilinear
+      // blocks take slope after slope: the registers of the other form leave two waves a SIMD in
+      // place of three (2x96^3: 328 us, 386 us with the loads together).
       const AdjGeo<GEO> G{a, B};
-      for (int d = 0; d < 3; ++d) {
-        const int64_t s = d == 0 ? 1 : (d == 1 ? (int64_t)B.sy : B.sz);
-        const int qd = p3[d];
-        for (int m = -1; m <= 1; ++m) {
-          const int qm = qd + m;
-          if (qm < 0 || qm > n3[d] + 1) continue;         // cells whose slope is never used
-          if (outside == 1 && (p3[d] >= 1 && p3[d] <= n3[d])) {
-            // a ghost cell of another direction: only its own slope along d could matter,
-            // and ghost cells never need a slope across the ghost layer
-            continue;
-          }
-          const int64_t cm = c + m * s;
-          double Spb[5], Smb[5];
-          bool any = false;
+      if constexpr (GEO == 1) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          const int64_t s = d == 0 ? 1 : (d == 1 ? (int64_t)B.sy : B.sz);
+          const int qd = p3[d], nd = n3[d];
+          // a ghost cell of another direction: ghost cells never need a slope across the ghost layer
+          if (outside == 1 && qd >= 1 && qd <= nd) continue;
+          if (adj_dead_dir(B, d)) continue;
+          bool use[3];                    // the slope of cell qd + m - 1 is used
+          double rl[4], hd[3];
+#pragma unroll
+          for (int m = 0; m < 3; ++m) use[m] = qd + m - 1 >= 0 && qd + m - 1 <= nd + 1;
+#pragma unroll
+          for (int m = 0; m < 4; ++m) rl[m] = (qd + m - 1 >= 0 && qd + m - 1 <= nd + 2) ? G.rl(d, c + (m - 1) * s, qd + m - 1) : 0.0;
+#pragma unroll
+          for (int m = 0; m < 3; ++m) hd[m] = use[m] ? G.hdl(d, c + (m - 1) * s, qd + m - 1) : 0.0;
+          double Sp[3][5], Sm[3][5], P[5][5];
 #pragma unroll
           for (int v = 0; v < 5; ++v) {
-            Spb[v] = a.W[(size_t)(10 * d + v) * N + cm];
-            Smb[v] = a.W[(size_t)(10 * d + 5 + v) * N + cm];
-            any = any || Spb[v] != 0.0 || Smb[v] != 0.0;
-          }
-          if (!any) continue;
-          double Pm[5], P0[5], Pp[5];
-          prim_load(a.Pp, N, cm - s, Pm);
-          prim_load(a.Pp, N, cm, P0);
-          prim_load(a.Pp, N, cm + s, Pp);
-          double bm[5] = {0, 0, 0, 0, 0}, b0[5] = {0, 0, 0, 0, 0}, bp[5] = {0, 0, 0, 0, 0};
-          double gb3[3] = {0.0, 0.0, 0.0};
-          const bool sp_geo = GEO == 1 && a.GL && m <= 0;
-          cell_states_adj<LIM>(Pm, P0, Pp, G.rl(d, cm, qm), G.rl(d, cm + s, qm + 1), G.hdl(d, cm, qm), Smb, Spb,
-                               bm, b0, bp, sp_geo ? gb3 : nullptr);
-          // rl(c) is rlm of c's own slope and rlp of the slope of c - e_d; hdl(c) = dl(c) / 2
-          if (m == 0) { rlb[d] += gb3[0]; dlb[d] += 0.5 * gb3[2]; }
-          else if (m == -1) rlb[d] += gb3[1];
-          const double* src = m == -1 ? bp : (m == 0 ? b0 : bm);
 #pragma unroll
-          for (int v = 0; v < 5; ++v) acc[v] += src[v];
+            for (int m = 0; m < 3; ++m) {
+              Sp[m][v] = use[m] ? a.W[(size_t)(10 * d + v) * N + c + (m - 1) * s] : 0.0;
+              Sm[m][v] = use[m] ? a.W[(size_t)(10 * d + 5 + v) * N + c + (m - 1) * s] : 0.0;
+            }
+#pragma unroll
+            for (int o = 0; o < 5; ++o)
+              P[o][v] = (qd + o - 2 >= -1 && qd + o - 2 <= nd + 2) ? a.Pp[(size_t)v * N + c + (o - 2) * s] : 0.0;
+          }
+          double g0 = 0.0, g1 = 0.0, g2 = 0.0;      // spacing adjoints: rlp of the low slope, rlm and hdl of the own
+#pragma unroll
+          for (int v = 0; v < 5; ++v) {
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+              // a slope that no face uses: its states may hold anything
+              if (Sp[m][v] == 0.0 && Sm[m][v] == 0.0) continue;
+              const double dm = P[m + 1][v] - P[m][v], dp = P[m + 2][v] - P[m + 1][v];
+              const double sm = dm * rl[m], sp = dp * rl[m + 1], gb = (Sp[m][v] - Sm[m][v]) * hd[m];
+              double spb = 0.0, smb = 0.0;
+              limiter_adj<LIM>(sp, sm, gb, spb, smb);
+              if (m == 0) acc[v] += spb * rl[1];
+              else if (m == 1) acc[v] += Sm[1][v] + Sp[1][v] - spb * rl[2] + smb * rl[1];
+              else acc[v] -= smb * rl[2];
+              if (GEO == 1 && a.GL) {
+                if (m == 0) g0 += spb * dp;
+                if (m == 1) { g1 += smb * dm; g2 += (Sp[1][v] - Sm[1][v]) * limiter<LIM>(sp, sm); }
+              }
+            }
+          }
+          // rl(c) is rlm of c's own slope and rlp of the slope of c - e_d; hdl(c) = dl(c) / 2
+          if (GEO == 1 && a.GL) {
+            rlb[d] += g0;
+            rlb[d] += g1;
+            dlb[d] += 0.5 * g2;
+          }
+        }
+      } else {
+        for (int d = 0; d < 3; ++d) {
+          const int64_t s = d == 0 ? 1 : (d == 1 ? (int64_t)B.sy : B.sz);
+          const int qd = p3[d];
+          if (adj_dead_dir(B, d)) continue;
+          for (int m = -1; m <= 1; ++m) {
+            const int qm = qd + m;
+            if (qm < 0 || qm > n3[d] + 1) continue;         // cells whose slope is never used
+            if (outside == 1 && (p3[d] >= 1 && p3[d] <= n3[d])) {
+              // a ghost cell of another direction: only its own slope along d could matter,
+              // and ghost cells never need a slope across the ghost layer
+              continue;
+            }
+            const int64_t cm = c + m * s;
+            double Spb[5], Smb[5];
+            bool any = false;
+#pragma unroll
+            for (int v = 0; v < 5; ++v) {
+              Spb[v] = a.W[(size_t)(10 * d + v) * N + cm];
+              Smb[v] = a.W[(size_t)(10 * d + 5 + v) * N + cm];
+              any = any || Spb[v] != 0.0 || Smb[v] != 0.0;
+            }
+            if (!any) continue;
+            double Pm[5], P0[5], Pp[5];
+            prim_load(a.Pp, N, cm - s, Pm);
+            prim_load(a.Pp, N, cm, P0);
+            prim_load(a.Pp, N, cm + s, Pp);
+            double bm[5] = {0, 0, 0, 0, 0}, b0[5] = {0, 0, 0, 0, 0}, bp[5] = {0, 0, 0, 0, 0};
+            double gb3[3] = {0.0, 0.0, 0.0};
+            const bool sp_geo = GEO == 1 && a.GL && m <= 0;
+            cell_states_adj<LIM>(Pm, P0, Pp, G.rl(d, cm, qm), G.rl(d, cm + s, qm + 1), G.hdl(d, cm, qm), Smb, Spb,
+                                 bm, b0, bp, sp_geo ? gb3 : nullptr);
+            // rl(c) is rlm of c's own slope and rlp of the slope of c - e_d; hdl(c) = dl(c) / 2
+            if (m == 0) { rlb[d] += gb3[0]; dlb[d] += 0.5 * gb3[2]; }
+            else if (m == -1) rlb[d] += gb3[1];
+            const double* src = m == -1 ? bp : (m == 0 ? b0 : bm);
+#pragma unroll
+            for (int v = 0; v < 5; ++v) acc[v] += src[v];
+          }
         }
       }
       // non-connection boundary faces naming this cell as boundary cell or neighbour
       if (outside == 0) {
         for (int f = 0; f < 6; ++f) {
-          if (B.bct[f] == F_CONN) continue;
+          if (B.bct[f] == F_CONN || B.bct[f] == F_NONE) continue;
           const int d = f >> 1, d1 = (d + 1) % 3, d2 = (d + 2) % 3;
           const bool fh = f & 1;
           const int nd = n3[d];

@@ -19,7 +19,8 @@ __global__ void __launch_bounds__(256) k_adj_prim(const double* __restrict__ U, 
   }
 }
 
-// Transpose of the ghost fill: each source cell adds M^T of the ghost adjoints it feeds.
+// Transpose of the ghost fill: each source cell adds M^T of the ghost adjoints it feeds (the steady and
+// march adjoints do it in their stage kernels instead, with ghost_bar).
 __global__ void __launch_bounds__(256) k_adj_ghostT(AdjArgs a) {
   const int64_t N = a.npool;
   for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < a.ngrows; q += gridDim.x * blockDim.x) {
@@ -496,7 +497,7 @@ __global__ void __launch_bounds__(256) k_adj_vbc(AdjArgs a) {
       }
       visc_vars_adj(P[m], Rg, Vb[m], Pb);
 #pragma unroll
-      for (int v = 0; v < 5; ++v) a.VBC[(10 * (int64_t)q + m) * 5 + v] = Pb[v];
+      for (int v = 0; v < 5; ++v) a.VBC[(int64_t)(5 * m + v) * a.nvf + q] = Pb[v];      // a row per value: coalesced
     }
     a.VB[q] = murefb;
   }
@@ -508,9 +509,9 @@ __global__ void __launch_bounds__(256) k_adj_vbc_gather(AdjArgs a) {
   for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < a.nvbt; r += gridDim.x * blockDim.x) {
     double acc[5] = {0, 0, 0, 0, 0};
     for (int64_t e = a.vbrow[r]; e < a.vbrow[r + 1]; ++e) {
-      const int64_t x = a.vbent[e];
+      const int x = a.vbent[e], q = x / 10, m = x - 10 * q;
 #pragma unroll
-      for (int v = 0; v < 5; ++v) acc[v] += a.VBC[x * 5 + v];
+      for (int v = 0; v < 5; ++v) acc[v] += a.VBC[(int64_t)(5 * m + v) * a.nvf + q];
     }
     const int64_t cell = a.vbt[r];
 #pragma unroll

@@ -15,6 +15,40 @@
 
 namespace mose {
 
+// What row `row` of the transposed ghost fill adds to its source cell (k_adj_ghostT without the
+// geometry part).
+__device__ __forceinline__ void ghost_bar(const AdjGhostRow* __restrict__ grows, const AdjGhostEnt* __restrict__ gents,
+                                          const double* __restrict__ Pbar, int64_t N, int row, double* acc) {
+  const AdjGhostRow R = grows[row];
+#pragma unroll
+  for (int v = 0; v < 5; ++v) acc[v] = 0.0;
+  for (int e = R.begin; e < R.end; ++e) {
+    const AdjGhostEnt E = gents[e];
+    double gb[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) gb[v] = Pbar[v * N + E.ghost];
+    if (E.kind == 0) {
+#pragma unroll
+      for (int v = 0; v < 5; ++v) acc[v] += E.w * gb[v];
+    } else {
+      const double dn = gb[1] * E.n[0] + gb[2] * E.n[1] + gb[3] * E.n[2];
+      acc[0] += gb[0];
+      acc[1] += gb[1] - 2.0 * dn * E.n[0];
+      acc[2] += gb[2] - 2.0 * dn * E.n[1];
+      acc[3] += gb[3] - 2.0 * dn * E.n[2];
+      acc[4] += gb[4];
+    }
+  }
+}
+
+// The transposed ghost fill taken by a stage kernel: row of each interior cell (-1: none); rows null
+// where k_adj_ghostT has run (a source of the fill is itself a ghost cell).
+struct GhostFold {
+  const int* __restrict__ rows;
+  const AdjGhostRow* __restrict__ grows;
+  const AdjGhostEnt* __restrict__ gents;
+};
+
 // One pseudo-time stage of the adjoint iteration over the interior cells.  Per cell c:
 //   x = gP - Pbar (the P-space adjoint residual, Pbar = (dR/dP)^T D lambda_in from the VJP),
 //   Q = (dP/dU)^T x at U*,
@@ -26,16 +60,18 @@ __global__ void __launch_bounds__(256) k_adjsolve_rk(const int64_t* __restrict__
                                                      const double* __restrict__ gP, const double* __restrict__ Pbar,
                                                      const double* lam0, const double* lamIn, double* lamOut,
                                                      double* __restrict__ Rbar, double a0, double b0, double gam,
-                                                     double* __restrict__ partial) {
+                                                     double* __restrict__ partial, GhostFold gf) {
   const double gm1 = gam - 1.0;
   double q2 = 0.0;
   for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x) {
     const int64_t c = cells[q];
-    double u[5], x[5], y[5];
+    double u[5], x[5], y[5], gb[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    const int row = gf.rows ? gf.rows[q] : -1;
+    if (row >= 0) ghost_bar(gf.grows, gf.gents, Pbar, N, row, gb);
 #pragma unroll
     for (int v = 0; v < 5; ++v) {
       u[v] = U[v * N + c];
-      x[v] = gP[v * N + c] - Pbar[v * N + c];
+      x[v] = gP[v * N + c] - (Pbar[v * N + c] + gb[v]);
     }
     const double ir = 1.0 / u[0];
     const double uu = u[1] * ir, vv = u[2] * ir, ww = u[3] * ir;

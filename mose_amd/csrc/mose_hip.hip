@@ -603,6 +603,11 @@ struct mose_ctx {
   double *d_gP = nullptr, *d_lam0 = nullptr, *d_lam1 = nullptr, *d_Dq = nullptr, *d_apart = nullptr;
   double* d_ares = nullptr;
   int64_t* d_icell = nullptr;                // interior pool cells
+  BcFace* d_adjbc = nullptr;                 // boundary faces with a flux (adjoint)
+  int nadjbc = 0;
+  std::vector<int64_t> grow_src;             // source cells of the transposed ghost fill, ascending
+  int* d_grow = nullptr;                     // row of each interior cell in it, or -1
+  bool fold_known = false;
   int64_t nicell = 0;
   // adjoint of the fixed-dt march (allocated on first use)
   std::vector<double> hvol;                  // volume of each interior cell (interior-list order)
@@ -1145,6 +1150,8 @@ static int ensure_adjoint(mose_ctx* c) {
     const BlockDev& B = c->lay.blocks[b];
     const int n[3] = {B.ni, B.nj, B.nk};
     for (int d = 0; d < 3; ++d) {
+      // no face of this direction is solved (adj_dead_dir)
+      if (n[d] == 1 && B.bct[2 * d] != F_CONN && B.bct[2 * d + 1] != F_CONN) continue;
       AdjSeg sg{};
       sg.start = start; sg.b = b; sg.d = d;
       sg.n0 = n[0] + (d == 0);
@@ -1201,6 +1208,13 @@ static int ensure_adjoint(mose_ctx* c) {
     r.end = (int)gents.size();
     grows.push_back(r);
   }
+  std::vector<BcFace> bcf;      // boundary faces with a flux
+  for (const BcFace& e : c->lay.bcfaces)
+    if (c->lay.blocks[e.b].bct[e.f] != F_NONE) bcf.push_back(e);
+  c->nadjbc = (int)bcf.size();
+  if (upload(c, &c->d_adjbc, bcf)) return c->err.code;
+  c->grow_src.clear();
+  for (const AdjGhostRow& r : grows) c->grow_src.push_back(r.src);
   c->ngrows = (int)grows.size();
   c->nents = (int)gents.size();
   if (upload(c, &c->d_segs, segs)) return c->err.code;
@@ -1241,14 +1255,29 @@ static int ensure_adjoint(mose_ctx* c) {
     row.push_back((int64_t)te.size());
     c->nvbt = (int)tgt.size();
     if (upload(c, &c->d_vbt, tgt) || upload(c, &c->d_vbrow, row) || upload(c, &c->d_vbent, ent)) return c->err.code;
-    // k_adj_visc: kVX x kVY patches of every viscous block, 32-plane chunks, i fastest
+    // k_adj_visc: kVX x kVY patches of every viscous block, i fastest.  One workgroup a CU (its LDS),
+    // each a serial chain of chunk + 2 planes, so the chunk of least rounds times (chunk + 2) is taken:
+    // 32 planes on two 96^3 boxes (216 patches), 4 on one of 40^3 (34 planes in 18 patches before).
+    int vkc = 32;
+    int64_t best = INT64_MAX;
+    for (int kc = 2; kc <= 64; ++kc) {
+      int64_t nt = 0;
+      int longest = 0;
+      for (const BlockDev& B : c->lay.blocks) {
+        if (!B.visc) continue;
+        nt += (int64_t)((B.ni + kVX - 1) / kVX) * ((B.nj + kVY - 1) / kVY) * ((B.nk + kc - 1) / kc);
+        longest = std::max(longest, std::min(kc, B.nk));
+      }
+      const int64_t ncu = std::max(c->ncu, 1), t = (nt + ncu - 1) / ncu * (longest + 2);
+      if (t < best) { best = t; vkc = kc; }
+    }
     std::vector<Tile> vt;
     for (int b = 0; b < c->nb; ++b) {
       const BlockDev& B = c->lay.blocks[b];
       if (!B.visc) continue;
-      for (int k0 = 1; k0 <= B.nk; k0 += 32)
+      for (int k0 = 1; k0 <= B.nk; k0 += vkc)
         for (int j0 = 1; j0 <= B.nj; j0 += kVY)
-          for (int i0 = 1; i0 <= B.ni; i0 += kVX) vt.push_back(Tile{b, i0, j0, k0, std::min(k0 + 32, B.nk + 1), 0, 0, 0});
+          for (int i0 = 1; i0 <= B.ni; i0 += kVX) vt.push_back(Tile{b, i0, j0, k0, std::min(k0 + vkc, B.nk + 1), 0, 0, 0});
     }
     c->nvtiles = (int)vt.size();
     if (upload(c, &c->d_vtiles, vt)) return c->err.code;
@@ -1282,9 +1311,9 @@ static AdjArgs adj_args(mose_ctx* c, const double* U = nullptr) {
   AdjArgs a{};
   a.U = U ? U : c->U[0]; a.Pp = c->d_Pp; a.Rbar = c->d_Rbar; a.W = c->d_W; a.BB = c->d_BB; a.Pbar = c->d_Pbar;
   a.blocks = c->d_blocks; a.lines = c->d_lines; a.geo = c->d_geo; a.facebc = c->d_facebc;
-  a.segs = c->d_segs; a.bcfaces = c->d_bcfaces; a.grows = c->d_grows; a.gents = c->d_gents;
+  a.segs = c->d_segs; a.bcfaces = c->d_adjbc; a.grows = c->d_grows; a.gents = c->d_gents;
   a.npool = c->npool; a.nwork = c->nwork; a.nslots = std::max<int64_t>(c->lay.nbcslots, 1);
-  a.nseg = c->nseg; a.nbcf = (int)c->lay.bcfaces.size(); a.ngrows = c->ngrows; a.nblocks = c->nb;
+  a.nseg = c->nseg; a.nbcf = c->nadjbc; a.ngrows = c->ngrows; a.nblocks = c->nb;
   a.nents = std::max(c->nents, 1);
   a.VW = c->d_VW; a.VB = c->d_VB; a.vfaces = c->d_vfaces; a.nvf = (int)c->lay.vfaces.size();
   a.VBC = c->d_VBC; a.Tp = c->d_Tp; a.vbt = c->d_vbt; a.vbrow = c->d_vbrow; a.vbent = c->d_vbent; a.nvbt = c->nvbt;
@@ -1312,11 +1341,17 @@ static int ensure_adjoint_geometry(mose_ctx* c) {
 // Pbar = (dR/dP)^T Rbar on the current state (the ghost layers are filled first); with
 // geometry, also the adjoints of the geometric quantities (face normals and areas, lengths,
 // mirror normals, inflow values).
-static void enqueue_vjp(mose_ctx* c, bool geometry = false, double* U = nullptr) {
-  if (!U) U = c->U[0];
+// prep: fill the ghost layers and form the primitives first (else a caller has, for the same state);
+// fold: leave the transposed ghost fill to the caller's stage kernel (ghost_fold).
+static void enqueue_adj_prep(mose_ctx* c, double* U) {
   enqueue_ghost(c, U);
   hipLaunchKernelGGL(k_adj_prim, dim3(launch_blocks(c->npool)), dim3(256), 0, c->stream, U, c->d_Pp, c->npool,
                      c->cfg.gamma, c->d_Tp, c->cfg.Rgas);
+}
+
+static void enqueue_vjp(mose_ctx* c, bool geometry = false, double* U = nullptr, bool prep = true, bool fold = false) {
+  if (!U) U = c->U[0];
+  if (prep) enqueue_adj_prep(c, U);
   AdjArgs a = adj_args(c, U);
   if (geometry) {
     a.GF = c->d_GF; a.GL = c->d_GL; a.BG = c->d_BG; a.GE = c->d_GE; a.IB = c->d_IB;
@@ -1341,8 +1376,9 @@ static void enqueue_vjp(mose_ctx* c, bool geometry = false, double* U = nullptr)
   } else {
     a.VPb = nullptr;
   }
-  (void)hipLaunchKernel((const void*)atable().face[lim][rs][geo], dim3(launch_blocks(c->nwork)), dim3(256), args, 0,
-                        c->stream);
+  if (c->nwork > 0)
+    (void)hipLaunchKernel((const void*)atable().face[lim][rs][geo], dim3(launch_blocks(c->nwork)), dim3(256), args, 0,
+                          c->stream);
   if (a.nbcf > 0)
     (void)hipLaunchKernel((const void*)atable().bc[lim][rs], dim3(launch_blocks(a.nbcf)), dim3(256), args, 0, c->stream);
   if (fork) (void)hipStreamWaitEvent(c->stream, c->ev_join, 0);
@@ -1357,7 +1393,7 @@ static void enqueue_vjp(mose_ctx* c, bool geometry = false, double* U = nullptr)
       hipLaunchKernelGGL(k_adj_vbc_gather, dim3(launch_blocks(a.nvbt)), dim3(256), 0, c->stream, a);
     }
   }
-  if (c->ngrows > 0)
+  if (c->ngrows > 0 && !fold)
     hipLaunchKernelGGL(k_adj_ghostT, dim3(launch_blocks(c->ngrows)), dim3(256), 0, c->stream, a);
 }
 
@@ -2036,6 +2072,27 @@ static int ensure_adjsolve(mose_ctx* c) {
   return 0;
 }
 
+// Row of each interior cell in the transposed ghost fill, for the stage kernels that take it along;
+// none where a source of the fill is a ghost cell (blocks one or two cells thick).
+static int ensure_fold(mose_ctx* c) {
+  if (c->fold_known) return 0;
+  std::vector<int> rows;
+  size_t r = 0;
+  for (const BlockDev& B : c->lay.blocks)
+    for (int k = 1; k <= B.nk; ++k)
+      for (int j = 1; j <= B.nj; ++j)
+        for (int i = 1; i <= B.ni; ++i) {
+          const int64_t cell = B.off + (i + 1) + (int64_t)B.sy * (j + 1) + B.sz * (k + 1);
+          const bool hit = r < c->grow_src.size() && c->grow_src[r] == cell;
+          rows.push_back(hit ? (int)r++ : -1);
+        }
+  if (r == c->grow_src.size() && r > 0 && upload(c, &c->d_grow, rows)) return c->err.code;
+  c->fold_known = true;
+  return 0;
+}
+
+static GhostFold ghost_fold(const mose_ctx* c) { return GhostFold{c->d_grow, c->d_grows, c->d_gents}; }
+
 int mose_put_objective_bar(mose_ctx* c, int32_t b, const double* gP) {
   if (!c || !c->finalized || b < 1 || b > c->nb || !gP) return fail(c, MOSE_E_ARG, b);
   if (ensure_adjoint(c) || ensure_adjsolve(c)) return c->err.code;
@@ -2101,19 +2158,26 @@ static int adjsolve_dt(mose_ctx* c) {
 
 // One pseudo-time iteration: n_rk stages, each a residual VJP of D lambda then the stage
 // update (k_adjsolve_rk); the first stage also forms |Q|^2 of the iteration's start.
+//
+// The state does not change: where the ghost fill depends on nothing but it (no cell of a previous fill),
+// the fill and the primitives are formed once a solve.  The sum of the |Q|^2 partials is taken
+// where the residual is looked at, and the transposed fill in the stage kernel: a stage is four launches
+// (seven or eight before, 102 us a stage on a 384x192 channel).
+static int adjsolve_grid(const mose_ctx* c) {
+  return (int)std::min<int64_t>(kAdjParts, std::max<int64_t>((c->nicell + 255) / 256, 1));
+}
 static void enqueue_adjsolve_iter(mose_ctx* c) {
   const int nrk = c->cfg.n_rk;
   const double cs3[3] = {1.0, 0.25, 2.0 / 3.0}, cs2[2] = {1.0, 0.5}, cs1[1] = {1.0};
   const double* cs = nrk == 3 ? cs3 : (nrk == 2 ? cs2 : cs1);
-  const int grid = (int)std::min<int64_t>(kAdjParts, std::max<int64_t>((c->nicell + 255) / 256, 1));
+  const int grid = adjsolve_grid(c);
   for (int s = 0; s < nrk; ++s) {
-    enqueue_vjp(c);
+    enqueue_vjp(c, false, nullptr, c->narc > 0, c->d_grow != nullptr);
     const double* lin = s == 0 ? c->d_lam0 : c->d_lam1;
     double* lout = s == nrk - 1 ? c->d_lam0 : c->d_lam1;
     hipLaunchKernelGGL(k_adjsolve_rk, dim3(grid), dim3(256), 0, c->stream, c->d_icell, c->d_Dq, c->nicell, c->npool,
                        c->U[0], c->d_gP, c->d_Pbar, c->d_lam0, lin, lout, c->d_Rbar, 1.0 - cs[s], cs[s],
-                       c->cfg.gamma, s == 0 ? c->d_apart : nullptr);
-    if (s == 0) hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(256), 0, c->stream, c->d_apart, grid, c->d_ares);
+                       c->cfg.gamma, s == 0 ? c->d_apart : nullptr, ghost_fold(c));
   }
 }
 
@@ -2121,7 +2185,7 @@ int mose_adjoint_solve(mose_ctx* c, int32_t max_iter, double rtol, int32_t check
                        double res[2]) {
   if (!c || !c->finalized || max_iter < 1 || check_every < 1 || !(rtol >= 0.0)) return fail(c, MOSE_E_ARG);
   if (c->err.code) return c->err.code;
-  if (ensure_adjoint(c) || ensure_adjsolve(c)) return c->err.code;
+  if (ensure_adjoint(c) || ensure_adjsolve(c) || ensure_fold(c)) return c->err.code;
   if (adjsolve_dt(c)) return c->err.code;
   const int64_t n5 = 5 * c->npool;
   for (double* p : {c->d_lam0, c->d_lam1, c->d_Rbar})
@@ -2134,11 +2198,13 @@ int mose_adjoint_solve(mose_ctx* c, int32_t max_iter, double rtol, int32_t check
     HIPCHK(c, hipGraphInstantiate(&c->agexec, c->agraph, nullptr, nullptr, 0));
   }
   c->vjp_valid = c->geo_valid = c->xbar_valid = false;
+  if (c->narc == 0) enqueue_adj_prep(c, c->U[0]);
   double r0 = 0.0, r = 0.0;
   int it = 0;
   while (it < max_iter) {
     const int n = it == 0 ? 1 : std::min(check_every, max_iter - it);
     for (int q = 0; q < n; ++q) HIPCHK(c, hipGraphLaunch(c->agexec, c->stream));
+    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(256), 0, c->stream, c->d_apart, adjsolve_grid(c), c->d_ares);
     it += n;
     if (const int rc = sync_and_check(c)) return rc;
     double a = 0.0;
@@ -2204,7 +2270,7 @@ static void enqueue_reverse_step(mose_ctx* c, double* Un) {
     const double cs = kRK[nrk - 1][s - 1];
     hipLaunchKernelGGL(k_unst_rbar, dim3(g), dim3(256), 0, c->stream, c->d_icell, c->d_Dq, c->nicell, c->npool,
                        c->d_lam0, c->d_lam1, c->d_Rbar, cs);
-    enqueue_vjp(c, false, in);
+    enqueue_vjp(c, false, in, true, c->d_grow != nullptr);
     if (c->lay.visc) {
       hipLaunchKernelGGL(k_mubar, dim3(kBlockParts, c->nb), dim3(256), 0, c->stream, c->d_blocks, c->d_VW, c->d_VB,
                          c->d_vfi, c->d_vfbeg, c->npool, c->d_upart);
@@ -2212,7 +2278,7 @@ static void enqueue_reverse_step(mose_ctx* c, double* Un) {
                          c->d_mu, 1);
     }
     hipLaunchKernelGGL(k_unst_back, dim3(g), dim3(256), 0, c->stream, c->d_icell, c->nicell, c->npool, in, c->d_Pbar,
-                       c->d_lam0, c->d_lam1, cs, c->cfg.gamma, s == 1 ? 1 : 0);
+                       c->d_lam0, c->d_lam1, cs, c->cfg.gamma, s == 1 ? 1 : 0, ghost_fold(c));
   }
   std::swap(c->d_lam0, c->d_lam1);       // dJ/dU_n is the next (earlier) step's result adjoint
   const int64_t n5 = 5 * c->npool;
@@ -2225,7 +2291,7 @@ int mose_unsteady_adjoint_ke(mose_ctx* c, int32_t nsteps, double dt, int32_t str
   if (!c->cfg.time_accurate || c->cfg.irs_beta > 0.0 || c->cfg.prim_vars) return fail(c, MOSE_E_ARG);
   const bool reverse = mu_bar != nullptr;
   if (reverse && ensure_adjoint(c)) return c->err.code;
-  if (ensure_unsteady(c)) return c->err.code;
+  if (ensure_unsteady(c) || (reverse && ensure_fold(c))) return c->err.code;
   {   // D = dt / vol
     std::vector<double> D(c->hvol.size());
     for (size_t q = 0; q < D.size(); ++q) D[q] = dt / c->hvol[q];
@@ -2386,7 +2452,7 @@ void mose_destroy(mose_ctx* c) {
                   c->d_GF, c->d_GL, c->d_BG, c->d_GE, c->d_IB, c->d_VW, c->d_VB, c->d_beta, c->d_pres, c->d_ghostp,
                   c->d_garc_cell, c->d_garc, c->d_gnrm, c->d_rs1, c->d_irsg, c->d_gP, c->d_lam0, c->d_lam1, c->d_Dq,
                   c->d_apart, c->d_ares, c->d_icell, c->d_VBC, c->d_Tp, c->d_vbt, c->d_vbrow, c->d_vbent, c->d_volq,
-                  c->d_upart, c->d_ke, c->d_mu, c->d_icbeg, c->d_vfbeg, c->d_vfi, c->d_vtiles, c->d_vghost, c->d_VPb};
+                  c->d_upart, c->d_ke, c->d_mu, c->d_icbeg, c->d_vfbeg, c->d_vfi, c->d_vtiles, c->d_vghost, c->d_VPb, c->d_adjbc, c->d_grow};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
   if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
