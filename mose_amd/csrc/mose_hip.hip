@@ -597,6 +597,8 @@ struct mose_ctx {
   hipGraphExec_t gexec = nullptr;
   hipGraph_t graph_n = nullptr;               // kStepsPerGraph steps in one graph (mose_advance)
   hipGraphExec_t gexec_n = nullptr;
+  hipGraph_t graph_l = nullptr;               // the last step of a call (with the norms)
+  hipGraphExec_t gexec_l = nullptr;
   // discrete adjoint (allocated on first use)
   bool adj_ready = false;
   // steady adjoint solve (allocated on first use)
@@ -964,8 +966,9 @@ static void enqueue_irs(mose_ctx* c, const StageArgs& a, bool last) {
 }
 
 // One explicit step enqueued on the context stream (no host synchronisation).  The CFL
-// time step of the next step is produced by the last RK stage from the state it writes.
-static int enqueue_step(mose_ctx* c) {
+// time step of the next step is produced by the last RK stage from the state it writes; with
+// norms, also the partial sums of the residual norms.
+static int enqueue_step(mose_ctx* c, bool norms) {
   const int nrk = c->cfg.n_rk;
   for (int s = 1; s <= nrk; ++s) {
     double* in = (s == 1) ? c->U[0] : c->U[s - 1];
@@ -978,7 +981,7 @@ static int enqueue_step(mose_ctx* c) {
       launch_stage(c, stage_fn(c, 2), r);        // R (prim) or R* = -R dt / vol into Rbuf
       enqueue_irs(c, a, s == nrk);
     } else {
-      launch_stage(c, stage_fn(c, s == nrk ? 1 : 0), a);
+      launch_stage(c, stage_fn(c, s < nrk ? 0 : (norms ? 1 : 3)), a);
     }
   }
   if (nrk == 1) {
@@ -1015,9 +1018,9 @@ static int sync_and_check(mose_ctx* c) {
 // of steps gives the same bits either way; the longer graph saves host launches on small cases,
 // whose steps are a few microseconds of work each).
 constexpr int kStepsPerGraph = 8;
-static int capture_steps(mose_ctx* c, int nsteps, hipGraph_t* graph, hipGraphExec_t* exec) {
+static int capture_steps(mose_ctx* c, int nsteps, bool norms, hipGraph_t* graph, hipGraphExec_t* exec) {
   HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-  for (int s = 0; s < nsteps; ++s) enqueue_step(c);
+  for (int s = 0; s < nsteps; ++s) enqueue_step(c, norms);
   const hipError_t le = hipGetLastError();
   HIPCHK(c, hipStreamEndCapture(c->stream, graph));
   if (le != hipSuccess) {
@@ -1032,8 +1035,9 @@ static int capture_steps(mose_ctx* c, int nsteps, hipGraph_t* graph, hipGraphExe
 
 static int ensure_graph(mose_ctx* c) {
   if (c->gexec) return 0;
-  if (capture_steps(c, 1, &c->graph, &c->gexec)) return c->err.code;
-  return capture_steps(c, kStepsPerGraph, &c->graph_n, &c->gexec_n);
+  if (capture_steps(c, 1, false, &c->graph, &c->gexec)) return c->err.code;
+  if (capture_steps(c, kStepsPerGraph, false, &c->graph_n, &c->gexec_n)) return c->err.code;
+  return capture_steps(c, 1, true, &c->graph_l, &c->gexec_l);
 }
 
 template <typename V>
@@ -1081,7 +1085,7 @@ static bool shape_compiled(const mose_ctx* c, int shape) {
 static int tile_launch_fits(mose_ctx* c) {
   const int nt = c->tx * c->ty;
   if (nt > kMaxTileThreads || nt % 64 != 0) return fail(c, MOSE_E_ARG);
-  const void* fns[] = {(const void*)stage_fn(c, 0), (const void*)stage_fn(c, 1), (const void*)stage_fn(c, 2),
+  const void* fns[] = {(const void*)stage_fn(c, 0), (const void*)stage_fn(c, 1), (const void*)stage_fn(c, 2), (const void*)stage_fn(c, 3),
                        (const void*)k_dt<0>, (const void*)k_dt<1>, (const void*)k_sd, (const void*)k_irs_jacobi,
                        (const void*)k_prim_resid<0>, (const void*)k_prim_resid<1>,
                        (const void*)k_irs_update<0, false, false>, (const void*)k_irs_update<0, true, false>,
@@ -1117,16 +1121,20 @@ static int retile(mose_ctx* c, int shape, int kchunk, int xcd) {
     HIPCHK(c, hipMalloc((void**)&c->d_partials, 5 * std::max<size_t>(nt, 1) * sizeof(double)));
   }
   c->grid_stage = (int)nt;
-  for (int m = 0; m < 3; ++m)     // occupancy queried here, never while a graph is captured
+  for (int m = 0; m < 4; ++m)     // occupancy queried here, never while a graph is captured
     if (StageFn fn = stage_fn(c, m)) (void)resident_per_cu(c, fn);
   if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
   if (c->graph) (void)hipGraphDestroy(c->graph);
   if (c->gexec_n) (void)hipGraphExecDestroy(c->gexec_n);
   if (c->graph_n) (void)hipGraphDestroy(c->graph_n);
+  if (c->gexec_l) (void)hipGraphExecDestroy(c->gexec_l);
+  if (c->graph_l) (void)hipGraphDestroy(c->graph_l);
   c->gexec = nullptr;
   c->graph = nullptr;
   c->gexec_n = nullptr;
   c->graph_n = nullptr;
+  c->gexec_l = nullptr;
+  c->graph_l = nullptr;
   if (c->agexec) (void)hipGraphExecDestroy(c->agexec);
   if (c->agraph) (void)hipGraphDestroy(c->agraph);
   c->agexec = nullptr;
@@ -1749,8 +1757,9 @@ int mose_advance(mose_ctx* c, int32_t nsteps, double* time_out, double* norms) {
     c->dt_primed = true;
   }
   int s = 0;
-  for (; s + kStepsPerGraph <= nsteps; s += kStepsPerGraph) HIPCHK(c, hipGraphLaunch(c->gexec_n, c->stream));
-  for (; s < nsteps; ++s) HIPCHK(c, hipGraphLaunch(c->gexec, c->stream));
+  for (; s + kStepsPerGraph < nsteps; s += kStepsPerGraph) HIPCHK(c, hipGraphLaunch(c->gexec_n, c->stream));
+  for (; s + 1 < nsteps; ++s) HIPCHK(c, hipGraphLaunch(c->gexec, c->stream));
+  if (nsteps > 0) HIPCHK(c, hipGraphLaunch(c->gexec_l, c->stream));
   // the norms of the last step (those of the steps before it are not observable)
   if (nsteps > 0)
     hipLaunchKernelGGL(k_normfin, dim3(1), dim3(256), 0, c->stream, c->d_partials, (int)c->lay.tiles.size(), c->d_scal);
@@ -2444,6 +2453,8 @@ void mose_destroy(mose_ctx* c) {
   if (c->graph) (void)hipGraphDestroy(c->graph);
   if (c->gexec_n) (void)hipGraphExecDestroy(c->gexec_n);
   if (c->graph_n) (void)hipGraphDestroy(c->graph_n);
+  if (c->gexec_l) (void)hipGraphExecDestroy(c->gexec_l);
+  if (c->graph_l) (void)hipGraphDestroy(c->graph_l);
   if (c->agexec) (void)hipGraphExecDestroy(c->agexec);
   if (c->agraph) (void)hipGraphDestroy(c->agraph);
   void* bufs[] = {c->U[0], c->U[1], c->U[2], c->Rbuf, c->stage, c->d_blocks, c->d_lines, c->d_geo, c->d_tiles,

@@ -27,6 +27,7 @@ void stage_modes(StageFn* t) {
   t[0] = k_stage<LIM, RS, FT, 0, TXc, TYc, GEO, SDR>;
   t[1] = k_stage<LIM, RS, FT, 1, TXc, TYc, GEO, SDR>;
   t[2] = k_stage<LIM, RS, FT, 2, TXc, TYc, GEO, SDR>;
+  t[3] = k_stage<LIM, RS, FT, 3, TXc, TYc, GEO, SDR>;
 }
 
 template <int LIM, int RS, int P, int GEO, int SH>

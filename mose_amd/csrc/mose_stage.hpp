@@ -323,7 +323,10 @@ __device__ __forceinline__ void stage_face(int d, int fi, int fj, int fk, const 
   }
 }
 
-// MODE 0: stage update; 1: last stage (update + residual-norm partials); 2: residual only.
+// MODE 0: stage update; 1: last stage (update + CFL time step + residual-norm partials); 2: residual
+// only; 3: last stage of a step whose norms nobody can read (every step of a call but its last): no
+// norms (2x128^3 viscous boxes, whose 128-thread patch then fits four times on a CU: last stage
+// 768 us with them, 527 us; 256^3, 32x16: 1184, 1171 us).
 // GEO 0: rectilinear blocks (geometry lines); 1: general metrics from the geometry arrays,
 // with face fluxes scaled by their areas where they are computed; 2: rectilinear blocks
 // with the laminar viscous terms (Fluxes_blk viscous sweeps, Mod_Fluxes.f90:101-207): the
@@ -375,11 +378,11 @@ __global__ void __launch_bounds__(TXc* TYc)
   constexpr int NL = (TXc > TYc ? TXc : TYc) + 3;
   __shared__ FT sRL[2][NL], sLP[2][NL];  // per-tile spacing data along x and y (rectilinear)
   __shared__ double sDel[2][NL], sDL[2][NL];   // node spacing delta and cell length dl along x, y
-  // last stage: the thread's residual-norm sums and least CFL time step, in LDS (the registers are
-  // full); reduced in a fixed order
+  // last stage: the thread's residual-norm sums, in LDS (the registers are full), reduced in a fixed
+  // order, and the least CFL time step of eight threads (bits of a positive double, LDS atomics)
+  constexpr bool LAST = MODE == 1 || MODE == 3;
   __shared__ double sN[5][MODE == 1 ? NTc : 1];
-  __shared__ double sDtT[MODE == 1 ? NTc : 1];
-  __shared__ double sDt[MODE == 1 ? NW : 1];
+  __shared__ unsigned long long sDtT[LAST ? NTc / 8 : 1];
   static_assert(NTc <= kMaxTileThreads, "tile shape above the helper kernels' launch bound");
 
   const int tid = threadIdx.x, tx = tid % TXc, ty = tid / TXc;
@@ -474,8 +477,10 @@ __global__ void __launch_bounds__(TXc* TYc)
     FT T1 = FT(0), T2 = FT(0);     // and the temperatures of Q1, Q2, from the FP64 state
 #pragma unroll
     for (int v = 0; v < 5; ++v) { Fkm_[v] = FT(0); Skp[v] = FT(0); Un3[v] = 0.0; Uh[v] = 0.0; }
+    if constexpr (LAST) {
+      if (tid < NTc / 8) sDtT[tid] = (unsigned long long)__double_as_longlong(1e300);
+    }
     if constexpr (MODE == 1) {
-      sDtT[tid] = 1e300;
 #pragma unroll
       for (int v = 0; v < 5; ++v) sN[v][tid] = 0.0;
     }
@@ -830,7 +835,7 @@ __global__ void __launch_bounds__(TXc* TYc)
             for (int v = 0; v < 5; ++v) bad = bad || (P[v] != P[v]);
             if (bad) set_error(a.err, MOSE_E_STATE, T.b + 1, i, j, k);
             if (P[0] < 1e-20) { P[0] = 1e-20; prim2cons(P, 1.0 / gm1, unew); }
-            if constexpr (MODE == 1) {
+            if constexpr (LAST) {
               // CFL time step of the new state for the next step (Compute_dt, Mod_dt.f90:61-85)
               const double snd = sqrt(a.gam * P[4] / P[0]);
               double dtc = 1e8;
@@ -853,7 +858,9 @@ __global__ void __launch_bounds__(TXc* TYc)
               const int itn = *a.iter + 1;
               if (itn < a.rampa) dtc = dtc * itn / a.rampa;
               if (a.local_dt) a.dtnext[c] = dtc;
-              sDtT[tid] = fmin(sDtT[tid], dtc);
+              atomicMin(&sDtT[tid >> 3], (unsigned long long)__double_as_longlong(dtc));
+            }
+            if constexpr (MODE == 1) {
               double pn[5];
               cons2prim(un, gm1, pn);
 #pragma unroll
@@ -923,9 +930,7 @@ __global__ void __launch_bounds__(TXc* TYc)
     if (more && tid == 0) sTile = claim_own(a.tq, a.nq, a.ntiles);
     lds_barrier();
 
-    if constexpr (MODE == 1) {   // fixed-order reductions over the workgroup: deterministic
-      double tot = 0.0;
-      double dtmin_t = sDtT[tid];
+    if constexpr (MODE == 1) {   // fixed-order reduction over the workgroup: deterministic
       for (int w = NTc / 2; w > 0; w >>= 1) {
         if (tid < w) {
 #pragma unroll
@@ -933,16 +938,15 @@ __global__ void __launch_bounds__(TXc* TYc)
         }
         lds_barrier();
       }
-      if (tid < 5) tot = sN[tid][0];
-      if (tid < 5) a.partials[5 * (int64_t)t + tid] = tot;
+      if (tid < 5) a.partials[5 * (int64_t)t + tid] = sN[tid][0];
+    }
+    if constexpr (LAST) {
       // one atomic a tile: every one goes to the same address, and 2048 of them (one a wave on the
       // 512x256 channel) made the last stage 46 us, now 26 us, where the others take 21 us
-      for (int o = 32; o > 0; o >>= 1) dtmin_t = fmin(dtmin_t, __shfl_xor(dtmin_t, o, 64));
-      if ((tid & 63) == 0) sDt[tid >> 6] = dtmin_t;
-      lds_barrier();
-      if (tid == 0) {
-        for (int w = 1; w < NW; ++w) dtmin_t = fmin(dtmin_t, sDt[w]);
-        if (dtmin_t < 1e300) atomicMin(a.dtmin, (unsigned long long)__double_as_longlong(dtmin_t));
+      if (tid < 64) {
+        double m = tid < NTc / 8 ? __longlong_as_double((long long)sDtT[tid]) : 1e300;
+        for (int o = 32; o > 0; o >>= 1) m = fmin(m, __shfl_xor(m, o, 64));
+        if (tid == 0 && m < 1e300) atomicMin(a.dtmin, (unsigned long long)__double_as_longlong(m));
       }
       lds_barrier();
     }

@@ -35,8 +35,8 @@ constexpr bool shape_built(int geo, int shape, bool detector) {
 
 // null where a variant is not compiled
 struct KTable {
-  StageFn f[3][2][NLIM][NRS][NSHAPE][3] = {};   // [geo][prec][lim][rs][shape][mode]
-  StageFn s[2][NLIM][NRS][3] = {};              // MUSCL-SD, FP64, tile shape 0: [geo 0/1][lim][rs][mode]
+  StageFn f[3][2][NLIM][NRS][NSHAPE][4] = {};   // [geo][prec][lim][rs][shape][mode]
+  StageFn s[2][NLIM][NRS][4] = {};              // MUSCL-SD, FP64, tile shape 0: [geo 0/1][lim][rs][mode]
   BcFn bc[2][NLIM][NRS] = {};
 };
 
