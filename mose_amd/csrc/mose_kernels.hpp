@@ -227,7 +227,9 @@ struct GhostArgs {
   const GhostRec* __restrict__ ops;
   const double* __restrict__ nrm;     // 3 per G_SYM record
   double* U;
-  const double* arc;
+  double* arc;
+  const int* save;             // 2 per record: archive slots of the two ghost cells it writes (-1: none); null
+                               // where the archive has a pass of its own, or there is none
   int64_t N, narc;
   double gam;
   int nops;
@@ -263,25 +265,28 @@ __device__ __forceinline__ void ghost_ops(const GhostArgs& g, int q0, int step) 
   if (q0 == 0 && g.dtmin) begin_step(g);
   const double gm1 = g.gam - 1.0, rgm1 = 1.0 / gm1;
   double* const U = g.U;
-  const double* const arc = g.arc;
+  double* const arc = g.arc;
   const int64_t N = g.N, narc = g.narc;
   for (int q = q0; q < g.nops; q += step) {
     const GhostRec op = g.ops[q];
     const int64_t d1 = op.b - op.s, d2 = op.b - 2 * (int64_t)op.s;
     auto rd = [&](int v, int64_t cell, int slot) { return slot >= 0 ? arc[v * narc + slot] : U[v * N + cell]; };
+    const int s1 = g.save ? g.save[2 * q] : -1, s2 = g.save ? g.save[2 * q + 1] : -1;
+    auto w1 = [&](int v, double x) { U[v * N + d1] = x; if (s1 >= 0) arc[v * narc + s1] = x; };
+    auto w2 = [&](int v, double x) { U[v * N + d2] = x; if (s2 >= 0) arc[v * narc + s2] = x; };
     if (op.type == G_COPY) {
 #pragma unroll
       for (int v = 0; v < 5; ++v) {
         const double a1 = rd(v, op.src1, op.a1), a2 = rd(v, op.src2, op.a2);
-        U[v * N + d1] = a1;
-        U[v * N + d2] = a2;
+        w1(v, a1);
+        w2(v, a2);
       }
     } else if (op.type == G_ZG) {
 #pragma unroll
       for (int v = 0; v < 5; ++v) {
         const double x = U[v * N + op.b];
-        U[v * N + d1] = x;
-        U[v * N + d2] = x;
+        w1(v, x);
+        w2(v, x);
       }
     } else if (op.type == G_EXTRAP) {
       double u[5], Pb[5], P1[5], P2[5], G1[5], G2[5];
@@ -301,10 +306,10 @@ __device__ __forceinline__ void ghost_ops(const GhostArgs& g, int q0, int step) 
       }
       ghost_cons(G1, rgm1, u);
 #pragma unroll
-      for (int v = 0; v < 5; ++v) U[v * N + d1] = u[v];
+      for (int v = 0; v < 5; ++v) w1(v, u[v]);
       ghost_cons(G2, rgm1, u);
 #pragma unroll
-      for (int v = 0; v < 5; ++v) U[v * N + d2] = u[v];
+      for (int v = 0; v < 5; ++v) w2(v, u[v]);
     } else {   // G_SYM: first layer only
       double u[5], P[5];
 #pragma unroll
@@ -317,7 +322,7 @@ __device__ __forceinline__ void ghost_ops(const GhostArgs& g, int q0, int step) 
       P[3] -= 2.0 * un * n[2];
       ghost_cons(P, rgm1, u);
 #pragma unroll
-      for (int v = 0; v < 5; ++v) U[v * N + d1] = u[v];
+      for (int v = 0; v < 5; ++v) w1(v, u[v]);
     }
   }
 }
