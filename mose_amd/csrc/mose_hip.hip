@@ -415,7 +415,7 @@ __global__ void __launch_bounds__(kMaxTileThreads) k_sd(SdArgs a) {
     if (i > B.ni || j > B.nj) continue;
     const int64_t sy = B.sy, sz = B.sz;
     const int64_t cbase = B.off + (int64_t)(i + 1) + sy * (j + 1);
-    for (int k = T.k0; k < T.k1; ++k) {
+    for (int k = T.k0 + (int)blockIdx.y; k < T.k1; k += (int)gridDim.y) {      // (gridDim.y: see k_irs_jacobi)
       const int64_t c = cbase + sz * (int64_t)(k + 1);
       a.beta[c] = sd_tramel(p[c], p[c - 1], p[c + 1], p[c - sy], p[c + sy], p[c - sz], p[c + sz]);
     }
@@ -825,7 +825,7 @@ static bool enqueue_ghost(mose_ctx* c, double* U, bool begin = false, const Stag
     hipLaunchKernelGGL(k_pres, dim3(launch_blocks(c->npool)), dim3(256), 0, c->stream, U, c->npool, c->cfg.gamma,
                        c->d_pres);
     SdArgs sa{c->d_pres, c->d_beta, c->d_tiles, c->d_blocks, c->npool, (int)c->lay.tiles.size(), c->tx, c->cfg.gamma};
-    hipLaunchKernelGGL(k_sd, dim3(sa.ntiles), dim3(c->tx * c->ty), 0, c->stream, sa);
+    hipLaunchKernelGGL(k_sd, dim3(sa.ntiles, std::min(c->kchunk, 64)), dim3(c->tx * c->ty), 0, c->stream, sa);
   }
   return bc_done;
 }
