@@ -825,7 +825,8 @@ static bool enqueue_ghost(mose_ctx* c, double* U, bool begin = false, const Stag
     hipLaunchKernelGGL(k_pres, dim3(launch_blocks(c->npool)), dim3(256), 0, c->stream, U, c->npool, c->cfg.gamma,
                        c->d_pres);
     SdArgs sa{c->d_pres, c->d_beta, c->d_tiles, c->d_blocks, c->npool, (int)c->lay.tiles.size(), c->tx, c->cfg.gamma};
-    hipLaunchKernelGGL(k_sd, dim3(sa.ntiles, std::min(c->kchunk, 64)), dim3(c->tx * c->ty), 0, c->stream, sa);
+    const dim3 planes(sa.ntiles, std::min(c->kchunk, 64));
+    hipLaunchKernelGGL(k_sd, planes, dim3(c->tx * c->ty), 0, c->stream, sa);
   }
   return bc_done;
 }
@@ -930,7 +931,7 @@ static IrsArgs irs_args(mose_ctx* c) {
 static void enqueue_irs(mose_ctx* c, const StageArgs& a, bool last) {
   IrsArgs ia = irs_args(c);
   const dim3 grid(ia.ntiles), block(c->tx * c->ty);
-  const unsigned ky = (unsigned)std::min(c->kchunk, 64);
+  const dim3 planes(ia.ntiles, std::min(c->kchunk, 64));      // a tile's planes over several workgroups
   ia.clamp = c->irs_clamp ? 1 : 0;
   const bool prim = c->cfg.prim_vars != 0, irs = c->cfg.irs_beta > 0.0;
   const int geo = c->lay.curvi ? 1 : (c->lay.visc ? 2 : 0);
@@ -951,7 +952,7 @@ static void enqueue_irs(mose_ctx* c, const StageArgs& a, bool last) {
       ia.d = d;
       ia.R = cur;
       ia.dst = nxt;
-      hipLaunchKernelGGL(k_irs_jacobi, dim3(ia.ntiles, ky), block, 0, c->stream, ia);
+      hipLaunchKernelGGL(k_irs_jacobi, planes, block, 0, c->stream, ia);
       std::swap(cur, nxt);
     }
     dl = c->ndir - 1;
@@ -960,7 +961,7 @@ static void enqueue_irs(mose_ctx* c, const StageArgs& a, bool last) {
   u.Rout = cur;
   const double b = c->cfg.irs_beta;
 #define MOSE_UPD(G, L, P) \
-  hipLaunchKernelGGL((k_irs_update<G, L, P>), dim3(ia.ntiles, L ? 1 : ky), block, 0, c->stream, u, tx, dl, b, ia.clamp)
+  hipLaunchKernelGGL((k_irs_update<G, L, P>), L ? grid : planes, block, 0, c->stream, u, tx, dl, b, ia.clamp)
   if (prim) {
     if (last) {
       if (geo == 1) MOSE_UPD(1, true, true);
