@@ -355,11 +355,6 @@ __global__ void __launch_bounds__(TXc* TYc)
   constexpr int NW = NTc / 64;                   // waves per workgroup
   constexpr int NH = 4 * (TXc + TYc);            // halo cells of a plane
   constexpr int NE = TXc + TYc;                  // faces on the high edges of the patch
-  constexpr bool VIS = GEO == 2;
-  // viscous FP32 stages: the ring's next plane comes from the column queue and from a halo prefetch
-  // that runs a plane further ahead, in place of loads that every thread waits for (2x128^3, 32x8:
-  // 394 us a stage with the loads, 341 us; in FP64 the registers that it takes spill, 499 to 545 us)
-  constexpr bool AHEAD = VIS && sizeof(FT) == 4;
   static_assert(NH <= NTc && NTc % 64 == 0, "one halo / edge cell per thread at most");
   __shared__ FT sP[5][TYc + 4][TXc + 4];
   // [y][x]: "+" i-state of cell x-1 (x = 0: the halo cell), then the flux of the low i face of
@@ -373,6 +368,7 @@ __global__ void __launch_bounds__(TXc* TYc)
   // moved too, or alone, 1.056 and 1.063 ms)
   constexpr bool KLDS = sizeof(FT) == 8 && GEO != 2;
   __shared__ FT sKm[5][KLDS ? NTc : 1];
+  constexpr bool VIS = GEO == 2;
   constexpr int VR = VIS ? 3 : 1, VY = VIS ? TYc + 2 : 1, VX = VIS ? TXc + 2 : 1;
   __shared__ FT sV[VR][4][VY][VX];       // viscous variables, ring over planes k-1, k, k+1
   constexpr int NL = (TXc > TYc ? TXc : TYc) + 3;
@@ -405,12 +401,6 @@ __global__ void __launch_bounds__(TXc* TYc)
   else if (tid < 4 * TYc) { const int h = tid - 2 * TYc; hy = h >> 1; hx = TXc + (h & 1); }
   else if (tid < 4 * TYc + 2 * TXc) { const int h = tid - 4 * TYc; hx = h % TXc; hy = -2 + h / TXc; }
   else if (tid < NH) { const int h = tid - 4 * TYc - 2 * TXc; hx = h % TXc; hy = TYc + h / TXc; }
-  // AHEAD: the four corner cells of the one-cell halo too (ring of viscous variables only),
-  // and whether this thread's halo cell belongs to that ring
-  static_assert(!AHEAD || NH + 4 <= NTc, "the corner cells take threads of their own");
-  const bool corner = AHEAD && tid >= NH && tid < NH + 4;
-  if (corner) { hx = (tid - NH) & 1 ? TXc : -1; hy = (tid - NH) & 2 ? TYc : -1; }
-  const bool ring = AHEAD && tid < NH + 4 && hx >= -1 && hx <= TXc && hy >= -1 && hy <= TYc;
   // the cells just outside the patch whose slopes are needed: the 2 TY x-halo cells by the
   // first lanes of wave 0, the 2 TX y-halo cells by the first lanes of wave 1
   static_assert(2 * TYc <= 64 && 2 * TXc <= 64 && NTc >= 128, "halo slope tasks: one wave per direction");
@@ -441,9 +431,7 @@ __global__ void __launch_bounds__(TXc* TYc)
     const int k0 = T.k0, k1 = T.k1;
     const bool offgrid = (k0 - 1) % kFp32Chunk != 0;      // FP32: see plus_state
     const int hgi = T.i0 + hx, hgj = T.j0 + hy;
-    const bool hin = hgi <= ni + 2 && hgj <= nj + 2;
-    const bool hval = tid < NH && hin;            // a halo cell of sP
-    const bool hload = (hval || corner) && hin;   // one whose state this thread loads
+    const bool hval = tid < NH && hgi <= ni + 2 && hgj <= nj + 2;
     const unsigned hbase = off + (unsigned)(hgi + 1) + (unsigned)sy_ * (unsigned)(hgj + 1);
     const int xci = T.i0 + xlx, xcj = T.j0 + xly, yci = T.i0 + ylx, ycj = T.j0 + yly;
     const bool xval = xtask && xcj <= nj && xci <= ni + 1;
@@ -473,8 +461,6 @@ __global__ void __launch_bounds__(TXc* TYc)
     // prefetched U(k+3) of the column and U of the next plane's halo cell
     FT Q0[5], Q1[5], Q2[5], Skp[5], Fkm_[5];
     double Un3[5], Uh[5];
-    FT Ph[5];                      // AHEAD: P of the halo cell at plane k (Uh: plane k + 1)
-    FT T1 = FT(0), T2 = FT(0);     // and the temperatures of Q1, Q2, from the FP64 state
 #pragma unroll
     for (int v = 0; v < 5; ++v) { Fkm_[v] = FT(0); Skp[v] = FT(0); Un3[v] = 0.0; Uh[v] = 0.0; }
     if constexpr (LAST) {
@@ -490,11 +476,6 @@ __global__ void __launch_bounds__(TXc* TYc)
       prim_at(Uin, N, cbase + sz * (unsigned)(k0), gm1, Q0);         // P(k0-1)
       prim_at(Uin, N, cbase + sz * (unsigned)(k0 + 1), gm1, Q1);     // P(k0)
       prim_at(Uin, N, cbase + sz * (unsigned)(k0 + 2), gm1, Q2);     // P(k0+1)
-      if constexpr (AHEAD) {
-        double p[5];
-        prim_at(Uin, N, cbase + sz * (unsigned)(k0 + 2), gm1, p);
-        T2 = p[0] != 0.0 ? (FT)(p[4] / (p[0] * a.R)) : FT(0);
-      }
       const unsigned cm = cbase + sz * (unsigned)(k0);            // cell k0-1
       FT bp = FT(1);
       if constexpr (SDR) bp = FT(beta[k0 >= 2 ? cm : cm + sz]);
@@ -514,13 +495,11 @@ __global__ void __launch_bounds__(TXc* TYc)
                                 FT(1), bp, Sm_, Skp);
       }
     }
-    if (hload) {
-      if constexpr (AHEAD) prim_at(Uin, N, hbase + sz * (unsigned)(k0 + 1), gm1, Ph);
+    if (hval) {
 #pragma unroll
-      for (int v = 0; v < 5; ++v) Uh[v] = Uin[v * N + hbase + sz * (unsigned)(k0 + (AHEAD ? 2 : 1))];
+      for (int v = 0; v < 5; ++v) Uh[v] = Uin[v * N + hbase + sz * (unsigned)(k0 + 1)];
     }
-    // viscous path: one-cell-halo plane kk of the viscous variables into ring slot (kk+3)%3 (AHEAD:
-    // the first two planes of the chunk only)
+    // viscous path: one-cell-halo plane kk of the viscous variables into ring slot (kk+3)%3
     const double Rgas = a.R;
     const FT Rg = FT(Rgas);
     auto stage_visc = [=](int kk) {
@@ -562,34 +541,7 @@ __global__ void __launch_bounds__(TXc* TYc)
 #pragma unroll
           for (int v = 0; v < 5; ++v) sP[v][ty + 2][tx + 2] = Q0[v];
         }
-        if constexpr (AHEAD) {
-          // the viscous variables of plane k + 1 from registers: the column's from its queue, the
-          // ring's from the halo prefetch, which runs one plane further ahead than the other stages'
-          const int slot = (k + 4) % 3;
-          const bool fl = colmem && Q1[0] != FT(0);
-#pragma unroll
-          for (int v = 0; v < 3; ++v) sV[slot][v][ty + 1][tx + 1] = fl ? Q1[1 + v] : FT(0);
-          sV[slot][3][ty + 1][tx + 1] = T1;
-          if (hval) {
-#pragma unroll
-            for (int v = 0; v < 5; ++v) sP[v][hy + 2][hx + 2] = Ph[v];
-          }
-          if (hload) {
-            double p[5];
-            cons2prim(Uh, gm1, p);
-#pragma unroll
-            for (int v = 0; v < 5; ++v) Ph[v] = (FT)p[v];
-            if (ring) {
-              const bool fh = p[0] != 0.0;
-#pragma unroll
-              for (int v = 0; v < 3; ++v) sV[slot][v][hy + 1][hx + 1] = fh ? (FT)p[1 + v] : FT(0);
-              sV[slot][3][hy + 1][hx + 1] = fh ? (FT)(p[4] / (p[0] * Rgas)) : FT(0);
-            }
-          } else if (ring) {      // beyond the block's padded extent
-#pragma unroll
-            for (int v = 0; v < 4; ++v) sV[slot][v][hy + 1][hx + 1] = FT(0);
-          }
-        } else if (hval) {
+        if (hval) {
           double p[5];
           cons2prim(Uh, gm1, p);
 #pragma unroll
@@ -601,13 +553,13 @@ __global__ void __launch_bounds__(TXc* TYc)
 #pragma unroll
         for (int v = 0; v < 5; ++v) Un3[v] = Uin[v * N + cbase + sz * (unsigned)(k + 4)];
       }
-      if (hload && plane && k + 1 < k1) {
+      if (hval && plane && k + 1 < k1) {
 #pragma unroll
-        for (int v = 0; v < 5; ++v) Uh[v] = Uin[v * N + hbase + sz * (unsigned)(k + (AHEAD ? 3 : 2))];
+        for (int v = 0; v < 5; ++v) Uh[v] = Uin[v * N + hbase + sz * (unsigned)(k + 2)];
       }
 
       if (plane) {
-        if constexpr (VIS && !AHEAD) stage_visc(k + 1);
+        if constexpr (VIS) stage_visc(k + 1);
         lds_barrier();       // plane k staged
 
         // ---- i and j face states: the own cell in each direction, then the cells just outside
@@ -920,10 +872,6 @@ __global__ void __launch_bounds__(TXc* TYc)
         cons2prim(Un3, gm1, p);
 #pragma unroll
         for (int v = 0; v < 5; ++v) { Q0[v] = Q1[v]; Q1[v] = Q2[v]; Q2[v] = (FT)p[v]; }
-        if constexpr (AHEAD) {
-          T1 = T2;
-          T2 = p[0] != 0.0 ? (FT)(p[4] / (p[0] * Rgas)) : FT(0);
-        }
       }
     }
     // the next tile (every thread has read sTile before the barriers of the planes)
