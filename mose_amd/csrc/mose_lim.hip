@@ -27,8 +27,9 @@ void stage_modes(StageFn* t) {
   t[0] = k_stage<LIM, RS, FT, 0, TXc, TYc, GEO, SDR>;
   t[1] = k_stage<LIM, RS, FT, 1, TXc, TYc, GEO, SDR>;
   t[2] = k_stage<LIM, RS, FT, 2, TXc, TYc, GEO, SDR>;
-  // without the norms the rectilinear FP32 last stage is the slower one (32 FP32 blocks: 421 us, 398 us with them)
-  if constexpr (sizeof(FT) == 4 && GEO == 0) t[3] = t[1];
+  // FP32 keeps the norms: the rectilinear stage is slower without them (32 FP32 blocks: 421 us, 398 us
+  // with them), and the viscous HLLC stage compiled without them rounds otherwise
+  if constexpr (sizeof(FT) == 4) t[3] = t[1];
   else t[3] = k_stage<LIM, RS, FT, 3, TXc, TYc, GEO, SDR>;
 }
 

@@ -324,8 +324,8 @@ __device__ __forceinline__ void stage_face(int d, int fi, int fj, int fk, const 
 }
 
 // MODE 0: stage update; 1: last stage (update + CFL time step + residual-norm partials); 2: residual
-// only; 3: last stage of a step whose norms nobody can read (every step of a call but its last): no
-// norms (2x128^3 viscous boxes, whose 128-thread patch then fits four times on a CU: last stage
+// only; 3: FP64, last stage of a step whose norms nobody can read (every step of a call but its last):
+// no norms (2x128^3 viscous boxes, whose 128-thread patch then fits four times on a CU: last stage
 // 768 us with them, 527 us; 256^3, 32x16: 1184, 1171 us).
 // GEO 0: rectilinear blocks (geometry lines); 1: general metrics from the geometry arrays,
 // with face fluxes scaled by their areas where they are computed; 2: rectilinear blocks

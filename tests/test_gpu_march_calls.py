@@ -33,6 +33,8 @@ CASES = {
     "box_fp32": lambda: perturb(cases.vortex(dims=(20, 17, 12), cfl=0.4, precision=abi.PREC_FP32_FLUX), seed=2),
     "viscous_fp64": lambda: perturb(cases.taylor_green(n=20, nbox=2), amp=0.01, seed=3),
     "viscous_fp32": lambda: perturb(cases.taylor_green(n=18, nbox=1, precision=abi.PREC_FP32_FLUX), amp=0.01, seed=4),
+    "viscous_fp32_hllc": lambda: perturb(cases.taylor_green(n=24, nbox=1, riemann="HLLC", precision=abi.PREC_FP32_FLUX),
+                                         amp=0.01, seed=5),
     "tube": lambda: cases.sod(n=70),
     "channel": lambda: cases.bump_channel(ni=40, nj=20, ncontrol=4, limiter="minmod"),
     "plane_0": lambda: _plane((37, 18, 1), [0, 0]),
