@@ -1429,6 +1429,10 @@ static void enqueue_residual(mose_ctx* c) {
   launch_stage(c, stage_fn(c, 2), a);
 }
 
+// Boundary-face fluxes that read their cell's inner neighbour (k_bcface): in a block one cell thick,
+// the first ghost cell of the opposite face.
+static bool bc_reads_neighbour(int bct) { return bct == F_SYM || bct == F_INFLOW || bct == F_INLET || bct == F_OUTFLOW; }
+
 // Fill phases and previous-fill archive of the ghost records.  The reference fills them one
 // record at a time in bc order (Fill_Ghost_Cell, Lib_Ghost.f90:11-137), so across a block one or
 // two cells thick an extrapolation (or a copy from such a donor) reads ghost cells of the
@@ -1474,18 +1478,23 @@ static int plan_ghost_fill(mose_ctx* c) {
   }
   // Records that no stage reads: zero-gradient ghost layers across a direction one cell thick with no
   // connection face.  That direction's faces take their fluxes from the boundary buffer, so its
-  // slopes go unused; the shock detector and the viscous terms do read the layers, and so
-  // does another record that extrapolates across the block (it is then archived, or there is a
+  // slopes go unused.  The layers are read, though, by the shock detector, by the viscous terms (of the
+  // block, and of a block connected to it: a viscous connection face takes the donor's tangential
+  // neighbours), by the boundary flux of the opposite face where that takes its cell's inner
+  // neighbour, and by another record that extrapolates across the block (it is then archived, or there is a
   // second phase).  They go last, and only the last step of a call fills them, for the caller: they
   // are 524,288 of the 527,360 ghost cells of the 512x256 channel (17.5 us a fill with all, 7.7 us).
-  std::vector<char> unread((size_t)n, 0);
+  std::vector<char> unread((size_t)n, 0), vdonor((size_t)c->nb, 0);
+  for (const mose_bc_entry& e : c->bc)
+    if ((e.type == 101 || e.type == 201) && c->lay.blocks[e.b - 1].visc) vdonor[e.bs - 1] = 1;
   if (np == 1 && !c->cfg.muscl_sd && !rs_takes_beta(c->cfg.riemann)) {
     for (int q = 0; q < n; ++q) {
       const mose_bc_entry& e = c->bc[q];
       const BlockDev& B = c->lay.blocks[e.b - 1];
       const int d = (e.f - 1) / 2, nd = d == 0 ? B.ni : (d == 1 ? B.nj : B.nk);
       const GhostOp& op = ops[q];
-      unread[q] = op.type == G_ZG && nd == 1 && !B.visc && B.bct[2 * d] != F_CONN && B.bct[2 * d + 1] != F_CONN &&
+      unread[q] = op.type == G_ZG && nd == 1 && !B.visc && !vdonor[e.b - 1] && B.bct[2 * d] != F_CONN &&
+                  B.bct[2 * d + 1] != F_CONN && !bc_reads_neighbour(B.bct[(e.f - 1) ^ 1]) &&
                   !slot.count(op.b - op.s) && !slot.count(op.b - 2 * op.s);
     }
   }
@@ -1539,8 +1548,7 @@ static int plan_ghost_fill(mose_ctx* c) {
   for (const BlockDev& B : c->lay.blocks) {
     const int n3[3] = {B.ni, B.nj, B.nk};
     for (int f = 0; f < 6; ++f)
-      if (n3[f / 2] < 2 && (B.bct[f] == F_SYM || B.bct[f] == F_INFLOW || B.bct[f] == F_INLET || B.bct[f] == F_OUTFLOW))
-        c->bc_indep = false;
+      if (n3[f / 2] < 2 && bc_reads_neighbour(B.bct[f])) c->bc_indep = false;
   }
   c->narc = (int64_t)cells.size();
   if (c->narc > 0) {
