@@ -681,16 +681,23 @@ static int fail(mose_ctx* c, int code, int b = 0, int i = 0, int j = 0, int k = 
   } while (0)
 
 // ---- state transfers between the caller's arrays and the device
-// A copy to or from pageable memory runs at about 10 GB/s (the 703 MB of a 256^3 state: 72 ms),
-// where the link carries 57 GB/s from pinned memory: one host thread copies between the runtime's
-// staging buffer and the caller's pages and takes their page faults.  Larger transfers are cut
+// A fetch into pageable memory runs at about 15 GB/s (10 GB/s into pages not yet touched: the 703 MB
+// of a 256^3 state took 72 ms) and an upload from it at 32 GB/s, where the link carries 57 GB/s from
+// pinned memory: one host thread copies between the runtime's staging buffer and the caller's pages
+// and takes their page faults.  Larger transfers are cut
 // into chunks that up to kXferThreads threads move through pinned chunk buffers, so the page
 // faults and copies of one overlap the link transfers of the others.  The buffers (32 MB) are
 // shared by all contexts of the process under a lock, allocated by the first such transfer and
 // freed with the last context.
+//
+// Starting and joining the threads takes 30 us (two) to 100 us (eight), so smaller transfers are one plain
+// copy.  The line lies where the two take the same time (plain, chunked): a residual adjoint, whose
+// fetch follows a few kernels, 291, 330 us with 1.8 MiB, 573, 586 us with 4.2, 779, 738 us with 6, 1434,
+// 1193 us with 12; uploads 131, 197 us at 3.3 MiB, 378, 464 us at 12, 940, 895 us at 32.
 constexpr int kXferThreads = 8;
 constexpr size_t kXferChunk = (size_t)4 << 20;
-constexpr size_t kXferMin = (size_t)1 << 20;      // below: one plain copy
+constexpr size_t kXferMinOut = (size_t)5 << 20, kXferMinIn = (size_t)28 << 20;
+constexpr size_t kXferPerThread = (size_t)1 << 20;      // at least, of a transfer cut up
 static std::mutex g_xfer_mu;
 static char* g_xfer_buf = nullptr;
 static int g_xfer_users = 0;                       // contexts alive
@@ -715,7 +722,7 @@ static hipError_t xfer(mose_ctx* c, void* dev, void* host, size_t n, bool to_hos
     const hipError_t e = to_host ? hipMemcpyAsync(host, dev, n, kind, c->stream) : hipMemcpyAsync(dev, host, n, kind, c->stream);
     return e != hipSuccess ? e : hipStreamSynchronize(c->stream);
   };
-  if (n < kXferMin) return plain();
+  if (n < (to_host ? kXferMinOut : kXferMinIn)) return plain();
   std::lock_guard<std::mutex> lock(g_xfer_mu);
   if (!g_xfer_buf && hipHostMalloc((void**)&g_xfer_buf, kXferThreads * kXferChunk, hipHostMallocPortable) != hipSuccess) {
     (void)hipGetLastError();
@@ -723,7 +730,7 @@ static hipError_t xfer(mose_ctx* c, void* dev, void* host, size_t n, bool to_hos
     return plain();
   }
   const int cpus = (int)std::max(1u, std::thread::hardware_concurrency());
-  const int nw = (int)std::min<size_t>((n + kXferMin - 1) / kXferMin, (size_t)std::min(kXferThreads, cpus));
+  const int nw = (int)std::min<size_t>((n + kXferPerThread - 1) / kXferPerThread, (size_t)std::min(kXferThreads, cpus));
   const size_t chunk = std::min(kXferChunk, ((n + nw - 1) / nw + 4095) & ~(size_t)4095);
   std::atomic<size_t> next{0};
   std::atomic<int> err{(int)hipSuccess};

@@ -1,0 +1,42 @@
+"""What a state transfer costs beside a plain copy of the same bytes."""
+import time
+
+import numpy as np
+import pytest
+
+from mose_amd import abi, cases
+
+pytestmark = pytest.mark.gpu
+
+
+def _least(fns, n=40):
+    """Least seconds of each of fns over n turns taken one after the other."""
+    out = [1e9] * len(fns)
+    for _ in range(n):
+        for q, f in enumerate(fns):
+            t0 = time.perf_counter()
+            f()
+            out[q] = min(out[q], time.perf_counter() - t0)
+    return out
+
+
+def test_mid_size_uploads_cost_a_plain_copy():
+    """Uploads of 1.3 to 12 MiB: the plain copy and the conversion kernel.  Through helper threads they took 1.4 times
+    as long in sum (764, 1188 us); half of that excess is allowed."""
+    import torch
+    from mose_amd.lib import GpuSolver
+    plain = put = 0.0
+    for n in (28, 32, 40, 50, 64):
+        g = GpuSolver(cases.vortex(dims=(n, n, n)))
+        P = np.random.default_rng(n).random(abi.padded_shape((n, n, n))) + 0.5
+        src, dst = torch.from_numpy(P), torch.empty(P.shape, dtype=torch.float64, device="cuda")
+
+        def copy():
+            dst.copy_(src)
+            torch.cuda.synchronize()
+
+        a, b = _least([copy, lambda: g.put_state(1, P)])
+        print("%d^3: copy %.1f us, put_state %.1f us" % (n, a * 1e6, b * 1e6))
+        plain, put = plain + a, put + b
+        g.close()
+    assert put < 1.2 * (plain + 5 * 15e-6), (plain, put)
