@@ -714,6 +714,17 @@ static void xfer_release() {
   }
 }
 
+// Memory that the runtime has allocated or registered (pinned, managed): a plain copy runs at the link's rate
+// there (32 MiB: 613 us up, 622 us down; through the chunk buffers 952 and 948 us).
+static bool runtime_knows(const void* p) {
+  hipPointerAttribute_t at{};
+  if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return at.type != hipMemoryTypeUnregistered;
+}
+
 // Copy of n bytes on the context's stream, after what is enqueued there; the host side is done on
 // return (device side: to_host only; else in stream order).
 static hipError_t xfer(mose_ctx* c, void* dev, void* host, size_t n, bool to_host) {
@@ -723,6 +734,7 @@ static hipError_t xfer(mose_ctx* c, void* dev, void* host, size_t n, bool to_hos
     return e != hipSuccess ? e : hipStreamSynchronize(c->stream);
   };
   if (n < (to_host ? kXferMinOut : kXferMinIn)) return plain();
+  if (runtime_knows(host)) return plain();
   std::lock_guard<std::mutex> lock(g_xfer_mu);
   if (!g_xfer_buf && hipHostMalloc((void**)&g_xfer_buf, kXferThreads * kXferChunk, hipHostMallocPortable) != hipSuccess) {
     (void)hipGetLastError();

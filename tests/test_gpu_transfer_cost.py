@@ -40,3 +40,26 @@ def test_mid_size_uploads_cost_a_plain_copy():
         plain, put = plain + a, put + b
         g.close()
     assert put < 1.2 * (plain + 5 * 15e-6), (plain, put)
+
+
+def test_pinned_arrays_are_copied_at_the_rate_of_the_link():
+    """States of 32 MiB: from and to pinned memory in 0.67 of the time that pageable memory takes (613 us up, 622 us
+    down; 940 and 948 us); through the chunk buffers they took as long."""
+    import ctypes as C
+
+    import torch
+    from mose_amd.lib import GpuSolver, _dp, load
+    L = load()
+    n = 90
+    g = GpuSolver(cases.vortex(dims=(n, n, n)))
+    P = np.random.default_rng(n).random(abi.padded_shape((n, n, n))) + 0.5
+    Q = np.empty_like(P)
+    pin = torch.empty(P.shape, dtype=torch.float64, pin_memory=True)
+    pin.copy_(torch.from_numpy(P))
+    pp = C.cast(C.c_void_p(pin.data_ptr()), C.POINTER(C.c_double))
+    put, put_pin = _least([lambda: L.mose_put_state(g.h, 1, _dp(P)), lambda: L.mose_put_state(g.h, 1, pp)], 15)
+    get, get_pin = _least([lambda: L.mose_get_state(g.h, 1, _dp(Q)), lambda: L.mose_get_state(g.h, 1, pp)], 15)
+    print("put %.1f us, pinned %.1f us; get %.1f us, pinned %.1f us" % (put * 1e6, put_pin * 1e6, get * 1e6, get_pin * 1e6))
+    assert np.array_equal(pin.numpy(), Q) and np.max(np.abs(Q - P)) < 1e-13
+    assert put_pin < 0.85 * put and get_pin < 0.85 * get
+    g.close()
