@@ -685,15 +685,18 @@ static int fail(mose_ctx* c, int code, int b = 0, int i = 0, int j = 0, int k = 
 // A fetch into pageable memory runs at about 15 GB/s (10 GB/s into pages not yet touched: the 703 MB
 // of a 256^3 state took 72 ms) and an upload from it at 32 GB/s, where the link carries 57 GB/s from
 // pinned memory: one host thread copies between the runtime's staging buffer and the caller's pages
-// and takes their page faults.  Larger transfers are cut
-// into chunks that up to kXferThreads threads move through pinned chunk buffers, so the page
-// faults and copies of one overlap the link transfers of the others.  The buffers (32 MB) are
-// shared by all contexts of the process, allocated by the first such transfer and
-// freed with the last context.  A worker has one for the length of a chunk, in the order of asking, so transfers
-// of contexts on other threads or devices run side by side; two chunks are on the link at a time, which keeps it
-// full and its queue short for the others.  Beside 88 MiB fetches a fetch of 1.8 MiB takes 128 us (127 us
-// alone; 0.1 to 0.6 ms with all eight chunks on the link), of 6 MiB 0.89 ms (0.34 ms) and of 32 MiB 1.5 ms
-// (0.95 ms); taking turns by the transfer, they took 2.2, 2.2 and 3.1 ms.
+// and takes their page faults.  Larger transfers are cut into chunks that up to kXferThreads threads
+// move through pinned chunk buffers, so the page faults and copies of one overlap the link transfers of
+// the others.  The buffers (32 MB) are shared by all contexts of the process, allocated by the first
+// such transfer and freed with the last context.
+//
+// A worker has a buffer for the length of a chunk, in the order of asking, so transfers of contexts on
+// other threads or devices run side by side.  Of a transfer with more chunks than workers, two chunks
+// are on the link at a time, which keeps it full and its queue short for the others.  Beside 88 MiB
+// fetches a fetch of 1.8 MiB takes 0.13 to 0.38 ms (0.13 ms alone; up to 0.6 ms with all eight chunks on
+// the link), of 6 MiB 0.61 ms (0.32 ms) and of 32 MiB 1.5 ms (0.95 ms); taking turns by the transfer,
+// they took 2.2, 2.2 and 3.1 ms.  (The chunks of shorter transfers are shorter than the hand-over: a
+// residual adjoint with 6 MiB took 830 us with two on the link, 750 us with all.)
 //
 // Starting and joining the threads takes 30 us (two) to 100 us (eight), so smaller transfers are one plain
 // copy.  The line lies where the two take the same time (plain, chunked): a residual adjoint, whose
@@ -781,6 +784,7 @@ static hipError_t xfer(mose_ctx* c, void* dev, void* host, size_t n, bool to_hos
   const int cpus = (int)std::max(1u, std::thread::hardware_concurrency());
   const int nw = (int)std::min<size_t>((n + kXferPerThread - 1) / kXferPerThread, (size_t)std::min(kXferThreads, cpus));
   const size_t chunk = std::min(kXferChunk, ((n + nw - 1) / nw + 4095) & ~(size_t)4095);
+  const bool queued = n > nw * chunk;
   std::atomic<size_t> next{0};
   std::atomic<int> err{(int)hipSuccess};
   auto work = [&](int w) {
@@ -798,12 +802,12 @@ static hipError_t xfer(mose_ctx* c, void* dev, void* host, size_t n, bool to_hos
       const int place = g_xfer_places.take();
       char* const pin = buf + (size_t)place * kXferChunk;
       if (!to_host) memcpy(pin, (char*)host + at, m);
-      const int link = g_xfer_link.take();
+      const int link = queued ? g_xfer_link.take() : 0;
       const bool sent = ok(to_host ? hipMemcpyAsync(pin, (char*)dev + at, m, kind, c->stream)
                                    : hipMemcpyAsync((char*)dev + at, pin, m, kind, c->stream)) &&
                         ok(hipEventRecord(ev, c->stream)) && ok(hipEventSynchronize(ev));
       if (!sent) (void)hipStreamSynchronize(c->stream);      // a copy in flight uses the buffer
-      g_xfer_link.give(link);
+      if (queued) g_xfer_link.give(link);
       if (sent && to_host) memcpy((char*)host + at, pin, m);
       g_xfer_places.give(place);
     }

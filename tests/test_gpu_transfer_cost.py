@@ -68,8 +68,8 @@ def test_pinned_arrays_are_copied_at_the_rate_of_the_link():
 
 @pytest.mark.parametrize("n", [32, 50])
 def test_a_small_transfer_does_not_wait_for_a_large_one(n):
-    """A context's fetches (2 and 6 MiB) beside another's 88 MiB fetches on a second thread: they share the link.
-    Taking turns, each waited 2.2 ms (16 and 7 times the time alone)."""
+    """A context's fetches (2 and 6 MiB) beside another's 88 MiB fetches on a second thread: they share the link
+    (0.13 to 0.4 and 0.6 to 0.9 ms).  Taking turns, each waited 2.2 ms."""
     from mose_amd.lib import GpuSolver, _dp, load
     L = load()
     small, large = GpuSolver(cases.vortex(dims=(n, n, n))), GpuSolver(cases.vortex(dims=(128, 128, 128)))
@@ -87,6 +87,7 @@ def test_a_small_transfer_does_not_wait_for_a_large_one(n):
         return sorted(t)[len(t) // 2]
 
     alone = median()
+    whole = _least([lambda: L.mose_get_state(large.h, 1, _dp(B))], 10)[0]
     stop = threading.Event()
 
     def loop():
@@ -101,6 +102,6 @@ def test_a_small_transfer_does_not_wait_for_a_large_one(n):
         stop.set()
         other.join()
     print("%d^3: alone %.1f us, beside %.1f us" % (n, alone * 1e6, beside * 1e6))
-    assert beside < 4.0 * alone
+    assert beside < alone + 0.5 * whole      # (a transfer that takes turns waits for a whole one)
     small.close()
     large.close()
