@@ -770,7 +770,9 @@ static hipError_t xfer(mose_ctx* c, void* dev, void* host, size_t n, bool to_hos
     return e != hipSuccess ? e : hipStreamSynchronize(c->stream);
   };
   if (n < (to_host ? kXferMinOut : kXferMinIn)) return plain();
-  if (runtime_knows(host)) return plain();
+  // the workers' events belong to the context's device, as its stream does
+  int dev_now = -1;
+  if (hipGetDevice(&dev_now) != hipSuccess || dev_now != c->dev || runtime_knows(host)) return plain();
   char* buf = nullptr;
   {
     std::lock_guard<std::mutex> lock(g_xfer_mu);
