@@ -242,8 +242,10 @@ int  mose_time_kernels(mose_ctx* ctx, int32_t nrep, double ms[4]);
 
 /* Autotuner: times the three stage launches of one step (on the current state, U^n not
  * modified) for every compiled tile shape, k-chunk of 8/16/32/64 planes and both tile orders
- * (linear, XCD-aware), keeps the fastest and re-captures the step with it.  choice (may be
- * NULL) receives {TX*1000+TY, k-chunk, xcd order}, best_ms the stage time of the winner
+ * (linear, XCD-aware), and re-captures the step with the fastest.  The tiling in use before the
+ * call stays where it is faster than all of them (small layouts, whose default has shorter
+ * chunks): mose_get_tiling tells which is in use.  choice (may be NULL) receives the fastest of
+ * those tried, {TX*1000+TY, k-chunk, xcd order}, best_ms its stage time
  * summed over the three launches.  No counterpart in the reference (its loops have fixed
  * OpenMP schedules). */
 int  mose_autotune(mose_ctx* ctx, int32_t nrep, int32_t choice[3], double* best_ms);

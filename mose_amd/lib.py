@@ -301,8 +301,9 @@ class GpuSolver:
                 "persistent": not bool(ch[2] & 2)}
 
     def autotune(self, nrep=3):
-        """Pick the fastest tile shape / k chunk / tile order by timing; returns
-        ({"tile": (TX, TY), "kchunk": kc, "xcd_order": bool}, ms of the three stage launches)."""
+        """Time the tile shapes / k chunks / tile orders and take the fastest, or stay with the tiling in
+        use where that is faster still (tiling() tells); returns the fastest of those tried,
+        ({"tile": (TX, TY), "kchunk": kc, "xcd_order": bool}, ms of its three stage launches)."""
         ch = np.zeros(3, dtype=np.int32)
         ms = np.zeros(1)
         self._check(load().mose_autotune(self.h, nrep, ch.ctypes.data_as(C.POINTER(C.c_int32)), _dp(ms)))
