@@ -1494,6 +1494,37 @@ static void enqueue_residual(mose_ctx* c) {
   launch_stage(c, stage_fn(c, 2), a);
 }
 
+// Number of each pool cell named, -1 for the others (open addressing; a std::map made three of these lookups
+// a third of the set-up of a 1000-cell tube).
+class CellIndex {
+ public:
+  explicit CellIndex(size_t most) {
+    size_t cap = 16;
+    while (cap < 2 * most) cap *= 2;
+    key_.assign(cap, -1);
+    val_.resize(cap);
+  }
+  int at(int64_t cell) const {
+    const size_t p = place(cell);
+    return key_[p] < 0 ? -1 : val_[p];
+  }
+  void set(int64_t cell, int v) {
+    const size_t p = place(cell);
+    key_[p] = cell;
+    val_[p] = v;
+  }
+
+ private:
+  size_t place(int64_t cell) const {
+    const size_t m = key_.size() - 1;
+    size_t p = ((uint64_t)cell * 0x9E3779B97F4A7C15ull >> 20) & m;
+    while (key_[p] >= 0 && key_[p] != cell) p = (p + 1) & m;
+    return p;
+  }
+  std::vector<int64_t> key_;
+  std::vector<int> val_;
+};
+
 // Boundary-face fluxes that read their cell's inner neighbour (k_bcface): in a block one cell thick,
 // the first ghost cell of the opposite face.
 static bool bc_reads_neighbour(int bct) { return bct == F_SYM || bct == F_INFLOW || bct == F_INLET || bct == F_OUTFLOW; }
@@ -1507,15 +1538,15 @@ static bool bc_reads_neighbour(int bct) { return bct == F_SYM || bct == F_INFLOW
 static int plan_ghost_fill(mose_ctx* c) {
   const std::vector<GhostOp>& G = c->lay.ghost;
   const int n = (int)G.size();
-  std::map<int64_t, int> writer;
+  CellIndex writer(2 * (size_t)n);
   for (int q = 0; q < n; ++q) {
-    writer[G[q].b - G[q].s] = q;
-    if (G[q].type != G_SYM) writer[G[q].b - 2 * G[q].s] = q;
+    writer.set(G[q].b - G[q].s, q);
+    if (G[q].type != G_SYM) writer.set(G[q].b - 2 * G[q].s, q);
   }
   std::vector<GhostOp> ops(G);
   std::vector<int> phase(n, 0);
   std::vector<int64_t> cells;
-  std::map<int64_t, int> slot;
+  CellIndex slot(2 * (size_t)n);      // archive slot of a cell
   int np = n > 0 ? 1 : 0;
   for (int q = 0; q < n; ++q) {
     GhostOp& op = ops[q];
@@ -1523,18 +1554,16 @@ static int plan_ghost_fill(mose_ctx* c) {
     if (op.type != G_COPY && op.type != G_EXTRAP) continue;   // zero-gradient, symmetry: the boundary cell only
     const int64_t rc[2] = {op.type == G_COPY ? op.src1 : op.b + op.s, op.type == G_COPY ? op.src2 : op.b + 2 * op.s};
     for (int r = 0; r < 2; ++r) {
-      auto it = writer.find(rc[r]);
-      if (it == writer.end() || it->second == q) continue;
-      if (it->second < q) {
-        phase[q] = std::max(phase[q], phase[it->second] + 1);
+      const int w = writer.at(rc[r]);
+      if (w < 0 || w == q) continue;
+      if (w < q) {
+        phase[q] = std::max(phase[q], phase[w] + 1);
       } else {
-        auto sit = slot.find(rc[r]);
-        int sl = (int)cells.size();
-        if (sit == slot.end()) {
-          slot[rc[r]] = sl;
+        int sl = slot.at(rc[r]);
+        if (sl < 0) {
+          sl = (int)cells.size();
+          slot.set(rc[r], sl);
           cells.push_back(rc[r]);
-        } else {
-          sl = sit->second;
         }
         (r == 0 ? op.a1 : op.a2) = sl;
       }
@@ -1560,7 +1589,7 @@ static int plan_ghost_fill(mose_ctx* c) {
       const GhostOp& op = ops[q];
       unread[q] = op.type == G_ZG && nd == 1 && !B.visc && !vdonor[e.b - 1] && B.bct[2 * d] != F_CONN &&
                   B.bct[2 * d + 1] != F_CONN && !bc_reads_neighbour(B.bct[(e.f - 1) ^ 1]) &&
-                  !slot.count(op.b - op.s) && !slot.count(op.b - 2 * op.s);
+                  slot.at(op.b - op.s) < 0 && slot.at(op.b - 2 * op.s) < 0;
     }
   }
   std::vector<GhostRec> sorted;
@@ -1587,23 +1616,26 @@ static int plan_ghost_fill(mose_ctx* c) {
   // An archived cell whose one writer runs in a later phase than all its readers is archived by that
   // writer (a 1000-cell tube: one launch of 3.6 us less in a stage of 19 us); a mirror writes no second layer
   bool late = !cells.empty();
-  std::map<int64_t, int> wr;
+  std::vector<int> wr(cells.size(), -1);      // writer of each archived cell
   for (int q = 0; q < n && late; ++q) {
     const int64_t d1 = ops[q].b - ops[q].s, d2 = ops[q].b - 2 * ops[q].s;
     for (int64_t d : {d1, d2}) {
       if (d == d2 && ops[q].type == G_SYM) continue;
-      if (slot.count(d) && !wr.emplace(d, q).second) late = false;
+      const int sl = slot.at(d);
+      if (sl < 0) continue;
+      if (wr[sl] >= 0) late = false;
+      wr[sl] = q;
     }
   }
   for (int q = 0; q < n && late; ++q)
     for (int a : {ops[q].a1, ops[q].a2})
-      if (a >= 0 && (!wr.count(cells[a]) || phase[wr[cells[a]]] <= phase[q])) late = false;
+      if (a >= 0 && (wr[a] < 0 || phase[wr[a]] <= phase[q])) late = false;
   if (late) {
     std::vector<int> save(2 * sorted.size(), -1);
     for (size_t r = 0; r < sorted.size(); ++r) {
       const int64_t d1 = sorted[r].b - (int64_t)sorted[r].s, d2 = d1 - sorted[r].s;
-      if (slot.count(d1)) save[2 * r] = slot[d1];
-      if (sorted[r].type != G_SYM && slot.count(d2)) save[2 * r + 1] = slot[d2];
+      save[2 * r] = slot.at(d1);
+      if (sorted[r].type != G_SYM) save[2 * r + 1] = slot.at(d2);
     }
     if (upload(c, &c->d_gsave, save)) return c->err.code;
   }
