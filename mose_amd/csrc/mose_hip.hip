@@ -700,11 +700,12 @@ static int fail(mose_ctx* c, int code, int b = 0, int i = 0, int j = 0, int k = 
 //
 // Starting and joining the threads takes 30 us (two) to 100 us (eight), so smaller transfers are one plain
 // copy.  The line lies where the two take the same time (plain, chunked): a residual adjoint, whose
-// fetch follows a few kernels, 291, 330 us with 1.8 MiB, 573, 586 us with 4.2, 779, 738 us with 6, 1434,
-// 1193 us with 12; uploads 131, 197 us at 3.3 MiB, 378, 464 us at 12, 940, 895 us at 32.
+// fetch follows a few kernels, 291, 330 us with 1.8 MiB, 573, 586 us with 4.2, 764 to 797, 703 to 799 us
+// with 6, 936, 824 to 922 us with 7.4 and 1415, 1200 us with 12; uploads 131, 197 us at 3.3 MiB, 378,
+// 464 us at 12, 940, 895 us at 32.
 constexpr int kXferThreads = 8;
 constexpr size_t kXferChunk = (size_t)4 << 20;
-constexpr size_t kXferMinOut = (size_t)5 << 20, kXferMinIn = (size_t)28 << 20;
+constexpr size_t kXferMinOut = (size_t)7 << 20, kXferMinIn = (size_t)28 << 20;
 constexpr int kXferOnLink = 2;
 constexpr size_t kXferPerThread = (size_t)1 << 20;      // at least, of a transfer cut up
 
@@ -761,12 +762,14 @@ static bool runtime_knows(const void* p) {
   return at.type != hipMemoryTypeUnregistered;
 }
 
-// Copy of n bytes on the context's stream, after what is enqueued there; the host side is done on
-// return (device side: to_host only; else in stream order).
+// Copy of n bytes on the context's stream, after what is enqueued there; the host side of a fetch is
+// done on return, that of an upload when the caller has synchronised the stream (it does after the
+// kernel that takes the bytes: waiting here as well cost 10 us of a 90 us upload).
 static hipError_t xfer(mose_ctx* c, void* dev, void* host, size_t n, bool to_host) {
   const hipMemcpyKind kind = to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice;
   auto plain = [&]() {
-    const hipError_t e = to_host ? hipMemcpyAsync(host, dev, n, kind, c->stream) : hipMemcpyAsync(dev, host, n, kind, c->stream);
+    if (!to_host) return hipMemcpyAsync(dev, host, n, kind, c->stream);
+    const hipError_t e = hipMemcpyAsync(host, dev, n, kind, c->stream);
     return e != hipSuccess ? e : hipStreamSynchronize(c->stream);
   };
   if (n < (to_host ? kXferMinOut : kXferMinIn)) return plain();
