@@ -754,6 +754,7 @@ static void xfer_release() {
 // Memory that the runtime has allocated or registered (pinned, managed): a plain copy runs at the link's rate
 // there (32 MiB: 613 us up, 622 us down; through the chunk buffers 952 and 948 us).
 static bool runtime_knows(const void* p) {
+  if (hipPeekAtLastError() != hipSuccess) return true;      // a launch was refused: sync_and_check is to see it
   hipPointerAttribute_t at{};
   if (hipPointerGetAttributes(&at, p) != hipSuccess) {
     (void)hipGetLastError();

@@ -18,7 +18,6 @@ KINDS = {
     "inflow": {"type": 405, "mach": 0.4, "T": 1.0, "p": 0.75, "alpha": 0.1, "beta": 0.3, "rel_fac": 1.0},
     "outflow": {"type": 406, "p": 0.7, "rel_fac": 1.0},
 }
-PERX = [{"type": 201, "bs": 1, "fs": 2}, {"type": 201, "bs": 1, "fs": 1}]
 NSTEPS = 4
 
 
@@ -30,11 +29,13 @@ def _box(dims, hi):
 
 
 def _thin(axis, lo, hi, riemann="HLLC", precision=abi.PREC_FP64):
-    """A block one cell thick along axis (1: j, 2: k), periodic in x, open in the remaining direction."""
-    dims = (19, 1, 11) if axis == 1 else (19, 11, 1)
-    size = (1.0, 0.3, 0.7) if axis == 1 else (1.0, 0.7, 0.3)
-    thin = [KINDS[lo], KINDS[hi]]
-    faces = PERX + (thin + [400, 400] if axis == 1 else [400, 400] + thin)
+    """A block one cell thick along axis (0: i, 1: j, 2: k), periodic in the next direction, open in the third."""
+    per, other = (axis + 1) % 3, (axis + 2) % 3
+    dims, size, faces = [1] * 3, [0.3] * 3, [400] * 6
+    dims[per], size[per], dims[other], size[other] = 19, 1.0, 11, 0.7
+    faces[2 * axis:2 * axis + 2] = [KINDS[lo], KINDS[hi]]
+    faces[2 * per:2 * per + 2] = [{"type": 201, "bs": 1, "fs": 2 * per + 2}, {"type": 201, "bs": 1, "fs": 2 * per + 1}]
+    dims, size = tuple(dims), tuple(size)
     cfg = abi.make_cfg(1.4, 1.0 / 1.4, 0.3, "vanleer", riemann, 3, True, precision=precision)
     case = cases.Case("thin", cfg, [_box(dims, size)], cases.bc_records([{"dims": dims, "faces": faces}]))
     return perturb(case, amp=0.02, seed=9)
@@ -65,10 +66,11 @@ def test_thin_direction_faces(lo, hi):
     _march(_thin(2, lo, hi), oracle={lo, hi} != {"sym", "extrap"})
 
 
-@pytest.mark.parametrize("lo,hi", [("none", "sym"), ("sym", "none"), ("inflow", "sym"), ("inlet", "outflow")])
+@pytest.mark.parametrize("lo,hi", [("none", "none"), ("none", "sym"), ("sym", "none"), ("inflow", "sym"), ("inlet", "outflow")])
 @pytest.mark.parametrize("riemann", ["HLLC", "HLLC+"])
-def test_thin_direction_faces_along_j(lo, hi, riemann):
-    _march(_thin(1, lo, hi, riemann))
+@pytest.mark.parametrize("axis", [0, 1])
+def test_thin_direction_faces_along_i_and_j(axis, lo, hi, riemann):
+    _march(_thin(axis, lo, hi, riemann))
 
 
 def test_viscous_block_beside_an_inviscid_plane():

@@ -46,11 +46,10 @@ def _compare(monkeypatch, case, least_tiles):
 
 @pytest.mark.parametrize("prec", PRECS)
 def test_many_more_tiles_than_workgroups(monkeypatch, prec):
-    """Uneven blocks; more tiles than any occupancy of 256 threads a workgroup allows (2048 threads a CU)."""
-    import torch
-    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    """Uneven blocks; more tiles than any occupancy of 256 threads a workgroup allows (2048 threads on each of 256
+    CUs)."""
     case = perturb(cases.multiblock_chain(nblocks=12, seed=21, lo=30, hi=70, precision=prec), amp=0.01, seed=1)
-    _compare(monkeypatch, case, 8 * cus + 1)
+    _compare(monkeypatch, case, 8 * 256 + 1)
 
 
 # one j tile a plane and block: 32 x 8 m x nk cells are m nk tiles of 32 x 8 x 1
