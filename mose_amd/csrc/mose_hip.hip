@@ -12,12 +12,14 @@
 //                      update (Lib_Newstate.f90:134-160) fused; the last stage also
 //                      produces the residual-norm partial sums (Mod_Diagnostic.f90:13-50)
 //                      and, from the state it writes, the CFL time step of the next step
-//                      (Compute_dt, Mod_dt.f90:10-107: wave-shuffle min, one atomic per wave) }
+//                      (Compute_dt, Mod_dt.f90:10-107: one atomic per tile) }
 // and once per call, for its last step:
 //   k_normfin  fixed-order sum of the partials, sqrt                (Mod_Explicit.f90:111-112)
 // k_dt computes the CFL time step directly when the state did not come from a step.
 // Copy_State (PO = P) needs no pass: U^n stays in its own buffer while the stages run.
 #include <hip/hip_runtime.h>
+#include <sys/mman.h>
+#include <unistd.h>
 
 #include <algorithm>
 #include <atomic>
@@ -693,21 +695,22 @@ static int fail(mose_ctx* c, int code, int b = 0, int i = 0, int j = 0, int k = 
 // A worker has a buffer for the length of a chunk, in the order of asking, so transfers of contexts on
 // other threads or devices run side by side.  Of a transfer with more chunks than workers, two chunks
 // are on the link at a time, which keeps it full and its queue short for the others.  Beside 88 MiB
-// fetches a fetch of 1.8 MiB takes 0.13 to 0.38 ms (0.13 ms alone; up to 0.6 ms with all eight chunks on
-// the link), of 6 MiB 0.61 ms (0.32 ms) and of 32 MiB 1.5 ms (0.95 ms); taking turns by the transfer,
-// they took 2.2, 2.2 and 3.1 ms.  (The chunks of shorter transfers are shorter than the hand-over: a
-// residual adjoint with 6 MiB took 830 us with two on the link, 750 us with all.)
+// fetches a fetch of 1.8 MiB takes 0.17 ms (0.13 ms alone; up to 0.6 ms with all eight chunks on the
+// link), of 6 MiB 0.59 ms (0.28 ms) and of 32 MiB 1.5 ms (0.90 ms); taking turns by the transfer, they
+// took 2.2, 2.2 and 3.1 ms.  (The chunks of shorter transfers are shorter than the hand-over: a residual
+// adjoint with 6 MiB took 830 us with two on the link, 750 us with all.)
 //
-// Starting and joining the threads takes 30 us (two) to 100 us (eight), so smaller transfers are one plain
-// copy.  The line lies where the two take the same time (plain, chunked): a residual adjoint, whose
-// fetch follows a few kernels, 291, 330 us with 1.8 MiB, 573, 586 us with 4.2, 764 to 797, 703 to 799 us
-// with 6, 936, 824 to 922 us with 7.4 and 1415, 1200 us with 12; uploads 131, 197 us at 3.3 MiB, 378,
-// 464 us at 12, 940, 895 us at 32.
+// Sharing a transfer costs some tens of microseconds, so smaller ones are one plain copy, and those a
+// little above the line go to few threads: a residual adjoint, whose fetch follows a few kernels, takes
+// 286 us plain with 1.8 MiB (289 and 317 us with 1 and 2 MiB a thread), 462 with 3.3 (483, 434), 574 with 4.2
+// (559, 504), 1420 with 12 (1160 both).  Pages not yet touched ask for more threads, since their
+// faults take longer than the copy: fetches of 32 blocks of 2 to 16 MiB take 34 ms plain, 18 ms with 1 MiB a
+// thread and 20 ms with 2.  Uploads: 131 us plain, 197 us chunked at 3.3 MiB, 378, 464 us at 12, 940, 895 us at 32.
 constexpr int kXferThreads = 8;
 constexpr size_t kXferChunk = (size_t)4 << 20;
-constexpr size_t kXferMinOut = (size_t)7 << 20, kXferMinIn = (size_t)28 << 20;
+constexpr size_t kXferMinOut = (size_t)2 << 20, kXferMinIn = (size_t)28 << 20;
+constexpr size_t kXferPerThread = (size_t)2 << 20, kXferPerThreadFresh = (size_t)1 << 20;      // at least
 constexpr int kXferOnLink = 2;
-constexpr size_t kXferPerThread = (size_t)1 << 20;      // at least, of a transfer cut up
 
 // Places taken and given back, granted in the order of asking.
 class Places {
@@ -734,6 +737,113 @@ class Places {
   unsigned free_;
   uint64_t asked_ = 0, granted_;
 };
+// What a thread that moves chunks keeps: an event of the device it works for.
+struct ChunkThread {
+  int dev = -1;
+  hipEvent_t ev = nullptr;
+  hipError_t on(int d) {
+    if (dev == d) return hipSuccess;
+    drop();
+    hipError_t e = hipSetDevice(d);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+    if (e == hipSuccess) dev = d;
+    return e;
+  }
+  void drop() {
+    if (dev >= 0) (void)hipEventDestroy(ev);
+    dev = -1;
+  }
+};
+
+// Host threads that share the chunks of transfers with their calling threads, a chunk at a time for the
+// transfer that has the fewest of them.  The first is started by the first chunked transfer, each of
+// the others by the one before it, so the caller begins with its own chunk at once; they wait for the
+// next transfer and end with the last context.
+class Helpers {
+ public:
+  explicit Helpers(int most) : most_((size_t)most) {}
+  // step(thread) here and on up to n helpers until it returns false; one that comes after the last chunk is
+  // not waited for
+  template <typename F>
+  void run(int n, F& step) {
+    Job j{[](void* f, ChunkThread& t) { return (*(F*)f)(t); }, &step, n, 0, false};
+    try {
+      std::lock_guard<std::mutex> lock(mu_);
+      jobs_.push_back(&j);
+      if (threads_.empty() && most_ > 0) start();
+    } catch (...) {      // no memory or no thread: those there and this one do the work
+    }
+    wake_.notify_all();
+    ChunkThread me;
+    while (step(me)) {
+    }
+    me.drop();
+    std::unique_lock<std::mutex> lock(mu_);
+    jobs_.erase(std::remove(jobs_.begin(), jobs_.end(), &j), jobs_.end());
+    left_.wait(lock, [&] { return j.active == 0; });
+  }
+  void stop() {
+    {
+      std::lock_guard<std::mutex> lock(mu_);
+      stop_ = true;
+    }
+    wake_.notify_all();
+    for (std::thread& t : threads_) t.join();      // (none is added once stop_ is set)
+    threads_.clear();
+    stop_ = false;
+  }
+
+ private:
+  struct Job {
+    bool (*step)(void*, ChunkThread&);
+    void* work;
+    int most, active;
+    bool done;
+  };
+  void start() {
+    threads_.reserve(most_);
+    threads_.emplace_back([this] { loop(); });
+  }
+  void loop() {
+    ChunkThread me;
+    std::unique_lock<std::mutex> lock(mu_);
+    if (!stop_ && threads_.size() < most_) {
+      try {
+        start();
+      } catch (...) {
+      }
+    }
+    while (!stop_) {
+      Job* j = nullptr;
+      for (Job* q : jobs_)
+        if (!q->done && q->active < q->most && (!j || q->active < j->active)) j = q;
+      if (!j) {
+        wake_.wait(lock);
+        continue;
+      }
+      ++j->active;
+      lock.unlock();
+      const bool more = j->step(j->work, me);
+      lock.lock();
+      if (!more) j->done = true;
+      if (--j->active == 0) left_.notify_all();
+    }
+    lock.unlock();
+    me.drop();
+  }
+  const size_t most_;
+  std::mutex mu_;
+  std::condition_variable wake_, left_;
+  std::vector<Job*> jobs_;
+  std::vector<std::thread> threads_;
+  bool stop_ = false;
+};
+// never destroyed: a program may end with contexts, and so with waiting helpers
+static Helpers& xfer_helpers() {
+  static Helpers* h = new Helpers(std::min(kXferThreads, (int)std::max(1u, std::thread::hardware_concurrency())) - 1);
+  return *h;
+}
+
 static Places g_xfer_places(kXferThreads), g_xfer_link(kXferOnLink);
 static std::mutex g_xfer_mu;
 static char* g_xfer_buf = nullptr;
@@ -746,6 +856,7 @@ static void xfer_retain() {
 static void xfer_release() {
   std::lock_guard<std::mutex> lock(g_xfer_mu);
   if (--g_xfer_users == 0 && g_xfer_buf) {
+    xfer_helpers().stop();
     (void)hipHostFree(g_xfer_buf);
     g_xfer_buf = nullptr;
   }
@@ -761,6 +872,16 @@ static bool runtime_knows(const void* p) {
     return false;
   }
   return at.type != hipMemoryTypeUnregistered;
+}
+
+// Whether the pages of host memory have been touched (four of them are looked at).
+static bool touched(const void* p, size_t n) {
+  const uintptr_t page = (uintptr_t)sysconf(_SC_PAGESIZE);
+  for (int q = 0; q < 4; ++q) {
+    unsigned char in = 1;
+    if (mincore((void*)(((uintptr_t)p + n / 8 + n / 4 * q) & ~(page - 1)), 1, &in) == 0 && !(in & 1)) return false;
+  }
+  return true;
 }
 
 // Copy of n bytes on the context's stream, after what is enqueued there; the host side of a fetch is
@@ -787,49 +908,34 @@ static hipError_t xfer(mose_ctx* c, void* dev, void* host, size_t n, bool to_hos
     buf = g_xfer_buf;
   }
   if (!buf) return plain();
-  const int cpus = (int)std::max(1u, std::thread::hardware_concurrency());
-  const int nw = (int)std::min<size_t>((n + kXferPerThread - 1) / kXferPerThread, (size_t)std::min(kXferThreads, cpus));
+  const size_t per = to_host && !touched(host, n) ? kXferPerThreadFresh : kXferPerThread;
+  const int nw = (int)std::min<size_t>((n + per - 1) / per, kXferThreads);
   const size_t chunk = std::min(kXferChunk, ((n + nw - 1) / nw + 4095) & ~(size_t)4095);
   const bool queued = n > nw * chunk;
   std::atomic<size_t> next{0};
   std::atomic<int> err{(int)hipSuccess};
-  auto work = [&](int w) {
+  auto step = [&](ChunkThread& t) {
     auto ok = [&](hipError_t e) {
       if (e != hipSuccess) err.store((int)e);
       return e == hipSuccess;
     };
-    hipEvent_t ev;
-    if (w > 0 && !ok(hipSetDevice(c->dev))) return;      // worker 0 is the caller
-    if (!ok(hipEventCreateWithFlags(&ev, hipEventDisableTiming))) return;
-    for (;;) {
-      const size_t at = next.fetch_add(chunk);
-      if (at >= n || err.load() != (int)hipSuccess) break;
-      const size_t m = std::min(chunk, n - at);
-      const int place = g_xfer_places.take();
-      char* const pin = buf + (size_t)place * kXferChunk;
-      if (!to_host) memcpy(pin, (char*)host + at, m);
-      const int link = queued ? g_xfer_link.take() : 0;
-      const bool sent = ok(to_host ? hipMemcpyAsync(pin, (char*)dev + at, m, kind, c->stream)
-                                   : hipMemcpyAsync((char*)dev + at, pin, m, kind, c->stream)) &&
-                        ok(hipEventRecord(ev, c->stream)) && ok(hipEventSynchronize(ev));
-      if (!sent) (void)hipStreamSynchronize(c->stream);      // a copy in flight uses the buffer
-      if (queued) g_xfer_link.give(link);
-      if (sent && to_host) memcpy((char*)host + at, pin, m);
-      g_xfer_places.give(place);
-    }
-    (void)hipEventDestroy(ev);
+    const size_t at = next.fetch_add(chunk);
+    if (at >= n || err.load() != (int)hipSuccess || !ok(t.on(c->dev))) return false;
+    const size_t m = std::min(chunk, n - at);
+    const int place = g_xfer_places.take();
+    char* const pin = buf + (size_t)place * kXferChunk;
+    if (!to_host) memcpy(pin, (char*)host + at, m);
+    const int link = queued ? g_xfer_link.take() : 0;
+    const bool sent = ok(to_host ? hipMemcpyAsync(pin, (char*)dev + at, m, kind, c->stream)
+                                 : hipMemcpyAsync((char*)dev + at, pin, m, kind, c->stream)) &&
+                      ok(hipEventRecord(t.ev, c->stream)) && ok(hipEventSynchronize(t.ev));
+    if (!sent) (void)hipStreamSynchronize(c->stream);      // a copy in flight uses the buffer
+    if (queued) g_xfer_link.give(link);
+    if (sent && to_host) memcpy((char*)host + at, pin, m);
+    g_xfer_places.give(place);
+    return sent;
   };
-  std::thread th[kXferThreads];
-  int started = 0;
-  try {
-    for (int w = 1; w < nw; ++w) {
-      th[w] = std::thread(work, w);
-      started = w;
-    }
-  } catch (...) {      // no more threads: those running and this one do the rest
-  }
-  work(0);
-  for (int w = 1; w <= started; ++w) th[w].join();
+  xfer_helpers().run(nw - 1, step);
   return (hipError_t)err.load();
 }
 static hipError_t xfer_out(mose_ctx* c, double* host, const double* dev, int64_t n) {
@@ -918,7 +1024,7 @@ static StageArgs stage_args(mose_ctx* c, const double* Uin, const double* Un, do
 }
 
 // Persistent stage launch: as many workgroups as the device holds at once (never more than
-// there are tiles); they take tiles from the queues (claim_tile) until all are done.
+// there are tiles); after its first tile each takes others from the queues until all are done.
 static int resident_per_cu(mose_ctx* c, StageFn fn) {
   auto it = c->resident.find((const void*)fn);
   if (it != c->resident.end()) return it->second;
@@ -1672,7 +1778,8 @@ static int plan_ghost_fill(mose_ctx* c) {
 // the columns a CU then holds (32x16: 1092 us against 1116 us for 32x8 on 256^3, 86 against 101 us
 // on 128x96x80, 42 against 54 us on the 512x256 channel); a 256-thread workgroup alone on its CU
 // takes 0.62 of it (5.8 us against 9.5 us).  FP32-flux and MUSCL-SD layouts keep shape 0, viscous
-// FP64 layouts take the 128-thread patch (three on a CU: 636 against 712 us on 2x128^3).  FP32-flux
+// FP64 layouts take the 128-thread patch (2x128^3, shape 2 against shape 0: 487 against 688 us a stage, and
+// 781 against 773 us for the one last stage of a call).  FP32-flux
 // layouts take a divisor of 32 planes: the stage then gives the bits of 32-plane chunks
 // (plus_state).
 static void pick_tiling(mose_ctx* c, int* shape, int* kchunk) {

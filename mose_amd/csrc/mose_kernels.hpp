@@ -213,7 +213,8 @@ __device__ __forceinline__ void set_error(int* err, int code, int b, int i, int 
 //
 // The device's record: pool cells as 32-bit indexes (npool is below 2^31 / 5) and the mirror
 // normal in an array of its own, 32 bytes in place of 80 -- the fill reads a record for the ten to
-// twenty values it moves (256^3 periodic block, 393,216 records: 29.8 us, now 26.3 us a fill).
+// twenty values it moves (256^3 periodic block, 393,216 records: fills one after the other 29.8 us, now
+// 26.3 us; between the stages of a march 38 us).
 struct GhostRec {
   int b, s;            // boundary cell, inward stride
   int src1, src2;

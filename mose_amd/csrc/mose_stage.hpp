@@ -60,7 +60,8 @@ __device__ __forceinline__ void cell_states_b(const FT* Pm, const FT* P0, const 
 // it is added (it has two uses there); the copies that form the states below a chunk's first plane
 // fuse the two operations.  The results of FP32 layouts are those of kFp32Chunk-plane chunks: a chunk that
 // starts on a multiple of kFp32Chunk planes keeps the fused form, any other takes the form of the
-// march, so a smaller chunk (a divisor) changes no bit.
+// march, so a smaller chunk (a divisor) changes no bit.  A longer one does: the 64-plane chunks that the
+// tuner also tries (a 256^3 step of 2.49 ms, 2.52 ms with 32) have plane 33 inside the march.
 constexpr int kFp32Chunk = 32;
 template <int LIM>
 __device__ __forceinline__ void plus_state(const float* Pm, const float* P0, const float* Pp, float rlm, float rlp,
@@ -344,8 +345,8 @@ __device__ __forceinline__ void stage_face(int d, int fi, int fj, int fk, const 
 // Occupancy floor: FP32 flux 3 waves per SIMD (2 for 512-thread patches, whose workgroup
 // brings two waves to every SIMD); FP64 2 (256 registers: without the floor some variants take
 // a few AGPRs beyond 256 and fall to one wave per SIMD); the viscous kernels 2 for the FP64
-// 128-thread patch (its 51 KB of LDS let three workgroups share a CU; the floor costs a few
-// spilled registers and is 16 % faster than one wave per SIMD), else none (the LDS of the
+// 128-thread patch (its LDS lets four workgroups share a CU, three with the norms; the floor costs a
+// few spilled registers and is 16 % faster than one wave per SIMD), else none (the LDS of the
 // 256-thread viscous patches allows one workgroup per CU).
 template <int LIM, int RS, typename FT, int MODE, int TXc, int TYc, int GEO, bool SDR>
 __global__ void __launch_bounds__(TXc* TYc)
