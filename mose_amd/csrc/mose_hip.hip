@@ -151,10 +151,11 @@ __global__ void __launch_bounds__(256) k_irs_ghost(const int64_t* __restrict__ p
 }
 
 // x / den with rden = 1 / den rounded: a product and one correction by its exact remainder (Markstein;
-// correctly rounded for a correctly rounded rden), in place of a division's fifteen instructions.
+// correctly rounded for a correctly rounded rden), in place of a division's fifteen instructions.  The last
+// one gives an infinite x the division's infinity (its remainder is none).
 __device__ __forceinline__ double div_by(double x, double den, double rden) {
   const double q = x * rden;
-  return __builtin_fma(__builtin_fma(-q, den, x), rden, q);
+  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-q, den, x), rden, q), den, x);
 }
 
 // Both Jacobi sweeps of one direction (pool stride st) at cell c, index q of n along it: the first
